@@ -9,13 +9,12 @@
 // after token; nsx_pos_advance moves it on inside the graph.
 //
 // KV cache layout: K and V each [n_kv][ctx_max][head_dim] fp32.
-// Attention is split over chunks of ATTN_CHUNK keys (one workgroup per kv
-// head and chunk, each handling the kv head's n_rep query heads), and a
-// combine kernel merges the chunks in chunk order together with the sink; a
-// layer whose keys always fit one chunk (a 128-key sliding window) finishes
-// in the chunk kernel.
+// Attention is split over the keys (one workgroup per kv head and split, each
+// handling the kv head's n_rep query heads), and a combine kernel merges the
+// splits together with the sink; a layer whose keys always fit one workgroup
+// (a 128-key sliding window) finishes in the split kernel.
 // Both grids are sized for ctx_max, so their shape does not depend on the
-// position; chunks past the current length return at once.
+// position; each workgroup takes its share of the keys up to it.
 #include "nsx_common.h"
 
 #include <algorithm>
@@ -25,9 +24,15 @@
 namespace {
 
 constexpr int ATTN_D = 64;        // head_dim (GPT-OSS)
-constexpr int ATTN_CHUNK = 128;   // keys per attention workgroup (two rounds of 64)
-constexpr int ATTN_THREADS = 256;
-constexpr int ATTN_MAX_REP = 16;  // query heads per kv head
+constexpr int ATTN_TILE = 16;     // keys per wave and matrix-core step
+constexpr int ATTN_NW = 4;        // waves of a split's workgroup
+constexpr int ATTN_FINAL_NW = 8;  // waves of the only workgroup of a kv head: a tile each at 128 keys
+constexpr int ATTN_FINAL_KEYS = 128;  // up to this many keys one workgroup per kv head does everything
+constexpr int ATTN_MAX_REP = 16;  // query heads per kv head (columns of the matrix-core step)
+// Splits of a kv head's keys: enough workgroups for two on each of the 256 CUs, at most what the combine
+// kernel's lanes hold, and none shorter than a tile per wave.
+constexpr int ATTN_MAX_SPLIT = 128;
+constexpr int ATTN_GRID = 512;
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -53,6 +58,18 @@ __device__ __forceinline__ float rope_elem(float x, float partner, int d, int p,
   s *= amp;
   const float ps = partner * s;
   return d < ATTN_D / 2 ? fmaf(x, c, -ps) : fmaf(x, c, ps);
+}
+
+// The same for the pair (element d < 32, element d + 32): one sine and cosine serve both.
+__device__ __forceinline__ void rope_pair(float& x0, float& x1, int p, float inv_freq, float amp) {
+  const float ang = (float)p * inv_freq;
+  float s, c;
+  sincosf(ang, &s, &c);
+  c *= amp;
+  s *= amp;
+  const float y0 = fmaf(x0, c, -(x1 * s));
+  x1 = fmaf(x1, c, x0 * s);
+  x0 = y0;
 }
 
 // One wave per row of the q | k | v block: bias, then rotary for q and k
@@ -90,195 +107,310 @@ __device__ __forceinline__ void attn_span(int p, int window, int& lo, int& total
   total = p + 1 - lo;
 }
 
-// Workgroup (kv head g, chunk c of ATTN_CHUNK keys): the chunk's attention
-// for the kv head's n_rep query heads. Wave w takes query heads w, w + 4,
-// ... (HPW = ceil(n_rep / 4) of them) and walks the chunk in rounds of 64
-// keys: the scores with one key per lane, a running softmax per head in
-// registers (wave max / sum), then the value sums with lane = (key group
-// kg = lane / 16, dimensions 4 * (lane % 16) ..+3) over keys kg, kg + 4, ...,
-// so a round's 64 value rows are 16 coalesced 16-byte loads per lane. The
-// four key groups are summed with two shuffles at the end.
-// part[(h * nchunk + c) * (D + 2)] = {m, l, acc[D]} for query head h.
-// FINAL (only ever one chunk: a sliding window or a cache of at most
-// ATTN_CHUNK keys): the workgroup also merges the sink and writes out[h].
+// Keys per split: the token's keys in equal parts, whole tiles for each of the workgroup's waves.
+__device__ __forceinline__ int attn_per(int total, int nsplit, int nw) {
+  const int step = ATTN_TILE * nw;
+  return ((total + nsplit - 1) / nsplit + step - 1) / step * step;
+}
+
+// Workgroup (kv head g, split c): the attention of the kv head's n_rep query
+// heads over the split's keys. The token's keys are cut into gridDim.y splits
+// of equal length (a multiple of one ATTN_TILE per wave), so the number of
+// partials to merge does not grow with the history; splits past the current
+// length return at once.
+//
+// Wave w takes key tiles w, w + NW, ... of the split and multiplies them by
+// all query heads at once with v_mfma_f32_16x16x4_f32 (exact fp32 products
+// and sums), so every key and value row is loaded once, by one wave:
+//   scores: A = the tile's 16 keys x 4 dimensions, B = 4 dimensions x 16
+//     query heads. Lane l holds key l % 16 and, of every 16 dimensions, the
+//     four from 4 (l / 16): a 16-byte load serves four instructions. D: lane l
+//     holds query head l % 16 and keys 4 (l / 16) .. + 3.
+//   values: the D layout of the scores is the B layout of the next product (4
+//     keys x 16 heads) when instruction r takes keys r, 4 + r, 8 + r, 12 + r;
+//     A = 16 dimensions x those keys, lane l key 4 (l / 16) + r, dimensions
+//     4 (l % 16) .. + 3, one per instruction: coalesced 16-byte loads. D of
+//     instruction dt: lane l holds head l % 16, dimensions 16 (l / 16) + 4 i + dt.
+// A running softmax per head in registers (maximum over the four lane groups
+// by two shuffles), the next tile's rows in flight during a tile's products.
+// The waves are merged in wave order through LDS.
+//
+// Bound: the cache rows (67 MB for 8 kv heads x 16384 keys: 10 us at the card's read rate); the
+// products take 1024 cycles of a SIMD's matrix core per tile, about a third of that. Measured at 64 / 8
+// heads, 16384 keys: 17.2 us (3.9 TB/s) against 33 for a kernel whose four waves each loaded every key row
+// and multiplied on the VALU; 128 keys in one workgroup 6.9 us against 12.7. A second tile in flight per
+// wave: 20.5 against 19.1 us for the call, so one.
+//
+// part: for query head h and split c the values acc[ATTN_D] at (h * nsplit +
+// c) * ATTN_D, and behind all of those (m, l) at (h * nsplit + c) * 2.
+// FINAL (one split covers every position: a sliding window or a cache of at
+// most ATTN_FINAL_KEYS keys): the workgroup also merges the sink and writes out[h].
 // ROPE: q is the token's raw q | k | v block; each workgroup adds the bias
-// and applies the rotary to its query heads itself, and the workgroup whose
-// chunk holds the token's position does the same for the token's k row, adds
-// v's bias and appends both to the cache before it reads any key (no other
-// workgroup reads that row), so no separate rotary + append launch is needed.
+// and applies the rotary to its query heads itself. The workgroup whose split
+// holds the token's position does the same for the token's k row, adds v's
+// bias and appends both to the cache; its own products take the two rows from
+// LDS (no other workgroup reads them), so no separate rotary + append launch is needed.
 struct RopeArgs {
   const float *bq, *bk, *bv, *inv_freq;
   float amp;
 };
-template <bool FINAL, int HPW, bool ROPE>
-__global__ __launch_bounds__(ATTN_THREADS) void attn_chunk_kernel(
-    const float* __restrict__ q, float* k_cache, float* v_cache, const int32_t* __restrict__ pos_ptr,
-    int64_t ctx_max, int window, float scale, int n_rep, int n_head, int nchunk, float* __restrict__ part,
-    const float* __restrict__ sinks, float* __restrict__ out, RopeArgs ra) {
-  constexpr int NW = ATTN_THREADS / 64;
-  __shared__ float qs[ATTN_MAX_REP][ATTN_D];
-  // each wave's key weights, key j at (j % 4) * 16 + j / 4: key group kg reads its 16 as 4 vectors
-  __shared__ float wl[NW][HPW][64];
+
+// rows of one key tile in a wave's registers
+struct AttnTile {
+  v4f k[ATTN_D / 16], v[4];
+};
+
+__device__ __forceinline__ void attn_lds_barrier() {  // LDS writes visible; the tile loads stay in flight
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <bool FINAL, bool ROPE, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_split_kernel(
+    const float* __restrict__ q, float* __restrict__ k_cache, float* __restrict__ v_cache,
+    const int32_t* __restrict__ pos_ptr, int64_t ctx_max, int window, float scale, int n_rep, int n_head, int nsplit,
+    float* __restrict__ part, const float* __restrict__ sinks, float* __restrict__ out, RopeArgs ra) {
+  constexpr int NT = 64 * NW, HALF = ATTN_D / 2;
+  constexpr int PAIRS = (ATTN_MAX_REP * HALF + NT - 1) / NT;  // (d, d + 32) pairs of the query heads per thread
+  __shared__ __align__(16) float qs[ATTN_MAX_REP][ATTN_D + 4];
+  __shared__ __align__(16) float own[2][ATTN_D];  // the token's k and v rows
+  __shared__ float sm[NW][ATTN_MAX_REP], sl[NW][ATTN_MAX_REP];
+  __shared__ __align__(16) float sacc[NW][ATTN_MAX_REP][ATTN_D];
   const int g = blockIdx.x, c = blockIdx.y, t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, i16 = lane & 15, kq = lane >> 4;
+  // loads that do not depend on the position go out first
+  float x0[PAIRS], x1[PAIRS], fr[PAIRS], b0[PAIRS] = {}, b1[PAIRS] = {};
+#pragma unroll
+  for (int u = 0; u < PAIRS; ++u) {
+    const int i = min(t + u * NT, n_rep * HALF - 1);
+    const int64_t at = ((int64_t)g * n_rep + i / HALF) * ATTN_D + i % HALF;
+    x0[u] = q[at];
+    x1[u] = q[at + HALF];
+    if constexpr (ROPE) {
+      fr[u] = ra.inv_freq[i % HALF];
+      if (ra.bq) {
+        b0[u] = ra.bq[at];
+        b1[u] = ra.bq[at + HALF];
+      }
+    }
+  }
+  float n0 = 0.f, n1 = 0.f, nf = 0.f;  // threads 0..31: the token's k pair; 64..127: its v element
+  if constexpr (ROPE) {
+    static_assert(NT >= 128, "the token's own rows take two waves");
+    if (t < HALF) {
+      const float* kr = q + ((int64_t)n_head + g) * ATTN_D;
+      n0 = kr[t];
+      n1 = kr[t + HALF];
+      nf = ra.inv_freq[t];
+      if (ra.bk) {
+        n0 += ra.bk[(int64_t)g * ATTN_D + t];
+        n1 += ra.bk[(int64_t)g * ATTN_D + t + HALF];
+      }
+    } else if (t >= 64 && t < 128) {
+      n0 = q[((int64_t)n_head + n_head / n_rep + g) * ATTN_D + t - 64];  // v rows follow the n_kv k rows
+      if (ra.bv) n0 += ra.bv[(int64_t)g * ATTN_D + t - 64];
+    }
+  }
   const int p = *pos_ptr;
   if (p < 0 || p >= ctx_max) return;
   int lo, total;
   attn_span(p, window, lo, total);
-  const int k0 = c * ATTN_CHUNK;
+  const int per = attn_per(total, FINAL ? 1 : nsplit, NW);
+  const int k0 = c * per;
   if (k0 >= total) return;  // past the current length
-  const int nk = min(ATTN_CHUNK, total - k0);
-  if constexpr (ROPE) {
-    for (int i = t; i < n_rep * ATTN_D; i += ATTN_THREADS) {
-      const int64_t r = (int64_t)g * n_rep + i / ATTN_D;
-      const int d = i % ATTN_D, dp = d ^ (ATTN_D / 2);
-      float x = q[r * ATTN_D + d], xp = q[r * ATTN_D + dp];
+  const int nk = min(per, total - k0), ntile = (nk + ATTN_TILE - 1) / ATTN_TILE;
+  const int rel = k0 + nk == total ? nk - 1 : -1;  // ROPE: the token's own key in this split
+  const float* kb = k_cache + ((int64_t)g * ctx_max + lo + k0) * ATTN_D + 4 * kq;
+  const float* vb = v_cache + ((int64_t)g * ctx_max + lo + k0) * ATTN_D + 4 * i16;
+  // a tile's rows; rows past the split's keys are clamped to its last key and get weight 0
+  auto load = [&](int tile, AttnTile& T) {
+    const int r0 = tile * ATTN_TILE;
+    const float* kr = kb + (int64_t)min(r0 + i16, nk - 1) * ATTN_D;
+#pragma unroll
+    for (int j = 0; j < ATTN_D / 16; ++j) T.k[j] = *(const v4f*)(kr + 16 * j);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) T.v[r] = *(const v4f*)(vb + (int64_t)min(r0 + 4 * kq + r, nk - 1) * ATTN_D);
+  };
+  AttnTile T[2];
+  load(min(wave, ntile - 1), T[0]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < PAIRS; ++u) {
+    const int i = t + u * NT;
+    if (i >= n_rep * HALF) break;
+    float y0 = x0[u], y1 = x1[u];
+    if constexpr (ROPE) {
       if (ra.bq) {
-        x += ra.bq[r * ATTN_D + d];
-        xp += ra.bq[r * ATTN_D + dp];
+        y0 += b0[u];
+        y1 += b1[u];
       }
-      qs[i / ATTN_D][d] = rope_elem(x, xp, d, p, ra.inv_freq, ra.amp);
+      rope_pair(y0, y1, p, fr[u], ra.amp);
     }
-    if (c == (total - 1) / ATTN_CHUNK && t < 2 * ATTN_D) {  // this chunk holds the token's own key
-      const int d = t & (ATTN_D - 1);
-      const int64_t at = ((int64_t)g * ctx_max + p) * ATTN_D + d;
-      if (t < ATTN_D) {
-        const float* kr = q + ((int64_t)n_head + g) * ATTN_D;
-        const int dp = d ^ (ATTN_D / 2);
-        float x = kr[d], xp = kr[dp];
-        if (ra.bk) {
-          x += ra.bk[(int64_t)g * ATTN_D + d];
-          xp += ra.bk[(int64_t)g * ATTN_D + dp];
+    qs[i / HALF][i % HALF] = y0;
+    qs[i / HALF][i % HALF + HALF] = y1;
+  }
+  if constexpr (ROPE) {
+    if (rel >= 0) {
+      const int64_t at = ((int64_t)g * ctx_max + p) * ATTN_D;
+      if (t < HALF) {
+        rope_pair(n0, n1, p, nf, ra.amp);
+        own[0][t] = n0;
+        own[0][t + HALF] = n1;
+        k_cache[at + t] = n0;
+        k_cache[at + t + HALF] = n1;
+      } else if (t >= 64 && t < 128) {
+        own[1][t - 64] = n0;
+        v_cache[at + t - 64] = n0;
+      }
+    }
+  }
+  attn_lds_barrier();
+  v4f qr[ATTN_D / 16];  // query head i16 (heads past n_rep repeat the last and are not stored)
+#pragma unroll
+  for (int j = 0; j < ATTN_D / 16; ++j) qr[j] = *(const v4f*)&qs[min(i16, n_rep - 1)][16 * j + 4 * kq];
+  float m = -INFINITY, l = 0.f;
+  v4f acc[4] = {};
+  auto step = [&](int tile, AttnTile& cur) {
+    const int r0 = tile * ATTN_TILE;
+    if constexpr (ROPE) {
+      if (rel >= r0 && rel < r0 + ATTN_TILE) {  // the token's own rows, which this launch appends
+        if (r0 + i16 == rel) {
+#pragma unroll
+          for (int j = 0; j < ATTN_D / 16; ++j) cur.k[j] = *(const v4f*)&own[0][16 * j + 4 * kq];
         }
-        k_cache[at] = rope_elem(x, xp, d, p, ra.inv_freq, ra.amp);
-      } else {
-        float x = q[((int64_t)n_head + n_head / n_rep + g) * ATTN_D + d];  // v rows follow the n_kv k rows
-        if (ra.bv) x += ra.bv[(int64_t)g * ATTN_D + d];
-        v_cache[at] = x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (min(r0 + 4 * kq + r, nk - 1) == rel) cur.v[r] = *(const v4f*)&own[1][4 * i16];
       }
     }
-  } else {
-    for (int i = t; i < n_rep * ATTN_D; i += ATTN_THREADS)
-      qs[i / ATTN_D][i % ATTN_D] = q[((int64_t)g * n_rep + i / ATTN_D) * ATTN_D + i % ATTN_D];
-  }
-  __syncthreads();  // q staged; the appended k / v rows visible to the workgroup's loads
-  const int wave = t >> 6, lane = t & 63, kg = lane >> 4, dq = lane & 15;
-  const float* kb = k_cache + ((int64_t)g * ctx_max + lo + k0) * ATTN_D;
-  const float* vb = v_cache + ((int64_t)g * ctx_max + lo + k0) * ATTN_D + 4 * dq;
-  float m[HPW], l[HPW];
-  v4f acc[HPW];
+    v4f s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < HPW; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
-    acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-  }
-  for (int r0 = 0; r0 < nk; r0 += 64) {
-    const int n = min(64, nk - r0);
-    const bool valid = lane < n;
-    // All of the round's loads go out together; rows past the round's keys
-    // are clamped to its last key and get weight 0.
-    const v4f* kr = (const v4f*)(kb + (int64_t)(r0 + (valid ? lane : n - 1)) * ATTN_D);
-    v4f kv[ATTN_D / 4];
+    for (int j = 0; j < ATTN_D / 16; ++j) {
 #pragma unroll
-    for (int d4 = 0; d4 < ATTN_D / 4; ++d4) kv[d4] = kr[d4];
-    v4f vd[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) vd[u] = *(const v4f*)(vb + (int64_t)(r0 + min(kg + 4 * u, n - 1)) * ATTN_D);
-#pragma unroll
-    for (int i = 0; i < HPW; ++i) {
-      const int h = wave + i * NW;
-      float e = 0.f, corr = 1.f;
-      if (h < n_rep) {
-        float a = 0.f;
-#pragma unroll
-        for (int d4 = 0; d4 < ATTN_D / 4; ++d4) {
-          const v4f qv = *(const v4f*)&qs[h][4 * d4];
-          a = fmaf(qv.x, kv[d4].x, a); a = fmaf(qv.y, kv[d4].y, a);
-          a = fmaf(qv.z, kv[d4].z, a); a = fmaf(qv.w, kv[d4].w, a);
-        }
-        const float sc = valid ? a * scale : -INFINITY;
-        const float mn = fmaxf(m[i], wave_max(sc));  // finite: lane 0 holds a key
-        e = valid ? expf(sc - mn) : 0.f;
-        corr = expf(m[i] - mn);  // 0 on the first round (m = -inf)
-        l[i] = fmaf(l[i], corr, wave_sum(e));
-        m[i] = mn;
-      }
-      acc[i] *= corr;
-      wl[wave][i][(lane & 3) * 16 + (lane >> 2)] = e;
+      for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][e], qr[j][e], s, 0, 0, 0);
     }
-    __builtin_amdgcn_wave_barrier();
+    float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < HPW; ++i) {
-#pragma unroll
-      for (int u4 = 0; u4 < 4; ++u4) {
-        const v4f e = *(const v4f*)&wl[wave][i][kg * 16 + 4 * u4];  // keys kg + 4 * (4 * u4 + 0..3)
-        acc[i] += e.x * vd[4 * u4];
-        acc[i] += e.y * vd[4 * u4 + 1];
-        acc[i] += e.z * vd[4 * u4 + 2];
-        acc[i] += e.w * vd[4 * u4 + 3];
-      }
+    for (int r = 0; r < 4; ++r) {
+      s[r] = r0 + 4 * kq + r < nk ? s[r] * scale : -INFINITY;
+      mx = fmaxf(mx, s[r]);
     }
-    __builtin_amdgcn_wave_barrier();  // reads done before the next round's writes
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    const float mn = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));  // finite: a tile holds a key
+    const float corr = expf(m - mn);                                // 0 on the first tile (m = -inf)
+    m = mn;
+    float ls = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s[r] = r0 + 4 * kq + r < nk ? expf(s[r] - mn) : 0.f;
+      ls += s[r];
+    }
+    l = fmaf(l, corr, ls);  // this lane group's keys; the groups are added at the end
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) acc[dt] *= corr;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[r][dt], s[r], acc[dt], 0, 0, 0);
+    }
+  };
+  for (int tile = wave; tile < ntile; tile += 2 * NW) {
+    if (tile + NW < ntile) load(tile + NW, T[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    step(tile, T[0]);
+    if (tile + NW >= ntile) break;
+    if (tile + 2 * NW < ntile) load(tile + 2 * NW, T[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    step(tile + NW, T[1]);
   }
-#pragma unroll
-  for (int i = 0; i < HPW; ++i) {
-    const int h = wave + i * NW;
-    if (h >= n_rep) continue;
-    v4f a = acc[i];
-#pragma unroll
-    for (int o = 16; o < 64; o <<= 1) {
-      a.x += __shfl_xor(a.x, o, 64);
-      a.y += __shfl_xor(a.y, o, 64);
-      a.z += __shfl_xor(a.z, o, 64);
-      a.w += __shfl_xor(a.w, o, 64);
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (i16 < n_rep) {
+    if (kq == 0) {
+      sm[wave][i16] = m;
+      sl[wave][i16] = l;
     }
-    if (kg != 0) continue;
-    const int hq = g * n_rep + h;
-    if constexpr (FINAL) {  // the combine kernel's arithmetic for a single chunk
-      const float sink = sinks ? sinks[hq] : -INFINITY;
-      const float M = fmaxf(sink, m[i]);
-      const float w = expf(m[i] - M);
-      const float Z = fmaf(w, l[i], sinks ? expf(sink - M) : 0.f);
-      *(v4f*)(out + (int64_t)hq * ATTN_D + 4 * dq) =
-          v4f{(w * a.x) / Z, (w * a.y) / Z, (w * a.z) / Z, (w * a.w) / Z};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *(v4f*)&sacc[wave][i16][16 * kq + 4 * i] = v4f{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+  }
+  attn_lds_barrier();
+  for (int i = t; i < n_rep * ATTN_D; i += NT) {
+    const int h = i / ATTN_D, d = i % ATTN_D, hq = g * n_rep + h;
+    const float sink = FINAL && sinks ? sinks[hq] : -INFINITY;
+    float M = sink;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, sm[w][h]);
+    float Z = FINAL && sinks ? expf(sink - M) : 0.f, a = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {  // (a wave without a tile has weight 0)
+      const float e = expf(sm[w][h] - M);
+      Z = fmaf(e, sl[w][h], Z);
+      a = fmaf(e, sacc[w][h][d], a);
+    }
+    if constexpr (FINAL) {
+      out[(int64_t)hq * ATTN_D + d] = a / Z;
     } else {
-      float* o = part + ((int64_t)hq * nchunk + c) * (ATTN_D + 2);
-      if (dq == 0) {
-        o[0] = m[i];
-        o[1] = l[i];
+      part[((int64_t)hq * nsplit + c) * ATTN_D + d] = a;
+      if (d == 0) {
+        float* ml = part + (int64_t)n_head * nsplit * ATTN_D + ((int64_t)hq * nsplit + c) * 2;
+        ml[0] = M;
+        ml[1] = Z;
       }
-      float* od = o + 2 + 4 * dq;  // 8-byte aligned only: scalar stores
-      od[0] = a.x;
-      od[1] = a.y;
-      od[2] = a.z;
-      od[3] = a.w;
     }
   }
 }
 
-// One wave per query head: merge the chunks in order with the sink
-// (softmax over [scores, sink], the sink column dropped).
-__global__ __launch_bounds__(64) void attn_combine_kernel(
+// One workgroup per query head: merge the live splits with the sink (softmax
+// over [scores, sink], the sink column dropped). Every wave forms all the
+// splits' weights (lane = split), then wave w sums the values of splits w,
+// w + 4, ... (lane = dimension) with all its loads in flight, and the four
+// sums meet in LDS: one round trip for (m, l), one for the values. Bound by
+// those two and the launch; at 128 chunks in one serial loop the first version
+// took 64 us, this one 4.0.
+__global__ __launch_bounds__(256) void attn_combine_kernel(
     const float* __restrict__ part, const float* __restrict__ sinks, const int32_t* __restrict__ pos_ptr,
-    int64_t ctx_max, int window, int nchunk, float* __restrict__ out) {
-  const int h = blockIdx.x, d = threadIdx.x;
+    int64_t ctx_max, int window, int n_head, int nsplit, int nw, float* __restrict__ out) {
+  constexpr int LPS = ATTN_MAX_SPLIT / 64;  // splits per lane
+  __shared__ float ws[ATTN_MAX_SPLIT];
+  __shared__ float red[4][ATTN_D];
+  const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const float2* ml = (const float2*)(part + (int64_t)n_head * nsplit * ATTN_D) + (int64_t)h * nsplit;
+  const float sink = sinks ? sinks[h] : -INFINITY;
   const int p = *pos_ptr;
   if (p < 0 || p >= ctx_max) return;
   int lo, total;
   attn_span(p, window, lo, total);
-  const int nc = (total + ATTN_CHUNK - 1) / ATTN_CHUNK;
-  const float* ph = part + (int64_t)h * nchunk * (ATTN_D + 2);
-  const float sink = sinks ? sinks[h] : -INFINITY;
+  const int per = attn_per(total, nsplit, nw), nc = (total + per - 1) / per;  // 1 <= nc <= nsplit
+  float2 v[LPS];
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) v[i] = ml[min(lane + 64 * i, nc - 1)];
   float M = sink;
-  for (int c = 0; c < nc; ++c) M = fmaxf(M, ph[(int64_t)c * (ATTN_D + 2)]);
-  float Z = sinks ? expf(sink - M) : 0.f, acc = 0.f;
-  for (int c = 0; c < nc; ++c) {
-    const float* pc = ph + (int64_t)c * (ATTN_D + 2);
-    const float w = expf(pc[0] - M);
-    Z = fmaf(w, pc[1], Z);
-    acc = fmaf(w, pc[2 + d], acc);
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) M = fmaxf(M, v[i].x);
+  M = wave_max(M);
+  float z = 0.f;
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) {
+    const float e = lane + 64 * i < nc ? expf(v[i].x - M) : 0.f;
+    if (wave == 0) ws[lane + 64 * i] = e;
+    z = lane + 64 * i < nc ? fmaf(e, v[i].y, z) : z;
   }
-  out[(int64_t)h * ATTN_D + d] = acc / Z;
+  const float Z = wave_sum(z) + (sinks ? expf(sink - M) : 0.f);
+  __syncthreads();
+  const float* pv = part + (int64_t)h * nsplit * ATTN_D + lane;
+  float a = 0.f;
+  for (int c0 = wave; c0 < nc; c0 += 4 * 16) {
+    float x[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[u] = pv[(int64_t)min(c0 + 4 * u, nc - 1) * ATTN_D];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (c0 + 4 * u < nc) a = fmaf(ws[c0 + 4 * u], x[u], a);
+  }
+  red[wave][lane] = a;
+  __syncthreads();
+  if (wave == 0) out[(int64_t)h * ATTN_D + lane] = ((red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane])) / Z;
 }
 
 __global__ void pos_advance_kernel(int32_t* pos, int32_t n) {
@@ -305,14 +437,20 @@ extern "C" int nsx_rope_kv_append(float* qkv, const float* q_bias, const float* 
   return NSX_OK;
 }
 
-extern "C" int64_t nsx_attn_workspace_bytes(int n_head, int head_dim, int64_t ctx_max) {
-  if (head_dim != ATTN_D || n_head <= 0 || ctx_max <= 0) return -1;
-  const int64_t nchunk = nsx_cdiv(ctx_max, ATTN_CHUNK);
-  return (int64_t)n_head * nchunk * (ATTN_D + 2) * (int64_t)sizeof(float);
+// Splits per kv head for a cache of ctx_max rows (window bounds the keys when positive).
+static int attn_splits(int n_kv, int64_t ctx_max, int window) {
+  const int64_t keys = window > 0 ? std::min<int64_t>(ctx_max, window) : ctx_max;
+  const int64_t fill = std::min<int64_t>(ATTN_MAX_SPLIT, nsx_cdiv(ATTN_GRID, n_kv));
+  return (int)std::min<int64_t>(nsx_cdiv(keys, ATTN_TILE * ATTN_NW), fill);
 }
 
-// Checks shared by both attention entry points, then the chunk launches
-// (and the combine unless one chunk covers every position).
+extern "C" int64_t nsx_attn_workspace_bytes(int n_head, int head_dim, int64_t ctx_max) {
+  if (head_dim != ATTN_D || n_head <= 0 || ctx_max <= 0) return -1;
+  return (int64_t)n_head * attn_splits(1, ctx_max, 0) * (ATTN_D + 2) * (int64_t)sizeof(float);
+}
+
+// Checks shared by both attention entry points, then the split launch (and
+// the combine unless one workgroup per kv head covers every position).
 static int attn_launch(const float* q, float* k_cache, float* v_cache, const float* sinks, int n_head, int n_kv,
                        int head_dim, const int32_t* pos, int64_t ctx_max, int window, float scale,
                        void* workspace, float* out, bool rope, const RopeArgs& ra, hipStream_t st) {
@@ -325,38 +463,29 @@ static int attn_launch(const float* q, float* k_cache, float* v_cache, const flo
   NSX_REQUIRE(q && k_cache && v_cache && pos && workspace && out, NSX_EINVAL, "null buffer");
   NSX_REQUIRE(((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) % 16 == 0, NSX_EINVAL,
               "q, the caches and out must be 16-byte aligned");
-  const int nchunk = (int)nsx_cdiv(ctx_max, ATTN_CHUNK);
-  // a sliding window bounds the keys: only its chunks can be live
-  const int live = window > 0 ? (int)std::min<int64_t>(nchunk, nsx_cdiv(window, ATTN_CHUNK)) : nchunk;
-  const int n_rep = n_head / n_kv;
-  const int hpw = (n_rep + ATTN_THREADS / 64 - 1) / (ATTN_THREADS / 64);
-  auto chunks = [&](auto final_tag, auto hpw_tag, auto rope_tag) {
+  const int n_rep = n_head / n_kv, nsplit = attn_splits(n_kv, ctx_max, window);
+  // a sliding window bounds the keys; up to ATTN_FINAL_KEYS of them one workgroup and no combine launch
+  const bool final_ = std::min<int64_t>(ctx_max, window > 0 ? window : ctx_max) <= ATTN_FINAL_KEYS;
+  auto split = [&](auto final_tag, auto rope_tag) {
     constexpr bool F = decltype(final_tag)::value;
-    hipLaunchKernelGGL((attn_chunk_kernel<F, decltype(hpw_tag)::value, decltype(rope_tag)::value>),
-                       dim3(n_kv, F ? 1 : live), dim3(ATTN_THREADS), 0, st, q, k_cache, v_cache, pos, ctx_max,
-                       window, scale, n_rep, n_head, nchunk, (float*)workspace, sinks, out, ra);
+    constexpr int NW = F ? ATTN_FINAL_NW : ATTN_NW;
+    hipLaunchKernelGGL((attn_split_kernel<F, decltype(rope_tag)::value, NW>), dim3(n_kv, F ? 1 : nsplit),
+                       dim3(64 * NW), 0, st, q, k_cache, v_cache, pos, ctx_max, window, scale, n_rep, n_head, nsplit,
+                       (float*)workspace, sinks, out, ra);
   };
-  auto by_rope = [&](auto final_tag, auto hpw_tag) {
-    if (rope) chunks(final_tag, hpw_tag, std::true_type{});
-    else chunks(final_tag, hpw_tag, std::false_type{});
+  auto by_rope = [&](auto final_tag) {
+    if (rope) split(final_tag, std::true_type{});
+    else split(final_tag, std::false_type{});
   };
-  auto by_hpw = [&](auto final_tag) {
-    switch (hpw) {
-      case 1: by_rope(final_tag, std::integral_constant<int, 1>{}); break;
-      case 2: by_rope(final_tag, std::integral_constant<int, 2>{}); break;
-      case 3: by_rope(final_tag, std::integral_constant<int, 3>{}); break;
-      default: by_rope(final_tag, std::integral_constant<int, 4>{}); break;
-    }
-  };
-  if (live == 1) {  // one chunk at any position: no partials, no combine launch
-    by_hpw(std::true_type{});
+  if (final_) {
+    by_rope(std::true_type{});
     NSX_LAUNCHED();
     return NSX_OK;
   }
-  by_hpw(std::false_type{});
+  by_rope(std::false_type{});
   NSX_LAUNCHED();
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(n_head), dim3(64), 0, st, (const float*)workspace, sinks, pos,
-                     ctx_max, window, nchunk, out);
+  hipLaunchKernelGGL(attn_combine_kernel, dim3(n_head), dim3(256), 0, st, (const float*)workspace, sinks, pos,
+                     ctx_max, window, n_head, nsplit, ATTN_NW, out);
   NSX_LAUNCHED();
   return NSX_OK;
 }

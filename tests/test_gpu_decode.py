@@ -112,6 +112,44 @@ def test_fused_attention_equals_two_calls(dev, window, heads):
                        attn_decode_qkv(q0, None, None, None, c, inv, amp, kv2, 0, None, window))
 
 
+@pytest.mark.parametrize("heads,window", [((5, 1), 0), ((16, 1), 0), ((16, 8), 0), ((16, 1), 129), ((8, 1), 1000),
+                                          ((8, 4), 128), ((3, 3), 20)])
+def test_attention_split_edges(dev, heads, window):
+    """The split kernel at the edges of its tiles (16 keys), waves (64) and splits: a cache of 9000
+    rows (up to 128 splits, most of them empty at the first positions), rows past the position
+    holding NaN, against the same attention in float64."""
+    from nurostream_amd.model.decode import DeviceKV, attn_decode_qkv, yarn_inv_freq
+    c = _cfg(n_head=heads[0], n_kv=heads[1], window=window)
+    H, G, R = c.n_head, c.n_head_kv, c.n_rep
+    ctx = 9000
+    g = torch.Generator().manual_seed(3)
+    kv = DeviceKV(1, c, ctx, dev)
+    K, V = (torch.randn(G, ctx, 64, generator=g).to(dev) for _ in range(2))
+    inv, amp = yarn_inv_freq(c, dev)
+    sinks = torch.randn(H, generator=g).to(dev)
+    for p in (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 1023, 1024, 4095, 4096, 8190, 8191, 8192, 8999):
+        qkv = torch.randn((H + 2 * G) * 64, generator=g).to(dev)
+        kv.k[0].fill_(float("nan"))
+        kv.v[0].fill_(float("nan"))
+        kv.k[0][:, :p], kv.v[0][:, :p] = K[:, :p], V[:, :p]
+        kv.pos.fill_(p)
+        out = attn_decode_qkv(qkv, None, None, None, c, inv, amp, kv, 0, sinks, window)
+        ang = (torch.tensor(float(p)) * inv.cpu()).double()  # the fp32 angle, as the kernel forms it
+        cos, sin = ang.cos() * amp, ang.sin() * amp
+        rows = qkv.cpu().double().reshape(-1, 64)
+        rot = torch.cat([rows[:, :32] * cos - rows[:, 32:] * sin, rows[:, 32:] * cos + rows[:, :32] * sin], 1)
+        first = max(0, p + 1 - window) if window else 0
+        keys = torch.cat([K[:, first:p].cpu().double(), rot[H:H + G, None]], 1)
+        vals = torch.cat([V[:, first:p].cpu().double(), rows[H + G:, None]], 1)
+        s = (rot[:H].reshape(G, R, 1, 64) * keys[:, None]).sum(-1) / 8.0
+        w = torch.softmax(torch.cat([s, sinks.cpu().double().reshape(G, R, 1)], -1), -1)[..., :-1]
+        ref = (w[..., None] * vals[:, None]).sum(2).reshape(H, 64)
+        # scores are fp32 sums of 64 products (|s| < 30): e^s is off by at most 30 * 64 * 2^-24 = 1.1e-4, in
+        # practice the root of that count; the outputs average such errors over the keys
+        assert rel_max(to_np(out), ref.numpy()) < 2e-5, p
+        assert torch.equal(kv.v[0][:, p].cpu(), qkv.cpu().reshape(-1, 64)[H + G:])
+
+
 def test_attention_position_outside_cache_writes_nothing(dev):
     """A position at or past the cache capacity leaves the caches and the output untouched."""
     from nurostream_amd.model.decode import DeviceKV, attn_decode, attn_decode_qkv, rope_kv_append, yarn_inv_freq
