@@ -100,6 +100,17 @@ int nsx_fused_gemv(int ggml_type, const void *raw, int64_t n_rows, int64_t K,
 int nsx_fused_gemv_ex(int ggml_type, const void *raw, int64_t n_rows, int64_t K,
                       const void *x, int x_dtype, int64_t T, float *y, const float *bias,
                       const float *resid, void *stream);
+/* nsx_fused_gemv_ex with a caller's workspace, in which calls of several tokens
+ * keep their activation terms for the matrix cores (products of the exact
+ * weight codes and of 33 significant bits of each activation, fp32 sums):
+ * nsx_gemv_workspace_bytes for the same arguments says how much (0: none is
+ * used). 16-byte aligned, need not be cleared, free for other use once the
+ * call's work on the stream is done; NULL: as nsx_fused_gemv_ex, on the
+ * VALU. No reference counterpart (the reference fuses one token). */
+int64_t nsx_gemv_workspace_bytes(int ggml_type, int64_t n_rows, int64_t K, int64_t T);
+int nsx_fused_gemv_ws(int ggml_type, const void *raw, int64_t n_rows, int64_t K,
+                      const void *x, int x_dtype, int64_t T, float *y, const float *bias,
+                      const float *resid, void *workspace, int64_t workspace_bytes, void *stream);
 /* nsx_fused_gemv_ex for one token whose input is the block norm of the
  * residual stream: y = resid + (W . h + bias) with h = rms_norm(x + r) * w,
  * the rms_norm of compute/ops.py:14-20 ahead of the QKV linear

@@ -16,8 +16,8 @@ from pathlib import Path
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libnsx.so"
-SOURCES = ("quant.hip", "moe.hip", "attn.hip", "reader.hip")
-HEADERS = ("nsx_common.h", "raw_dot.h")
+SOURCES = ("quant.hip", "gemv_mm.hip", "moe.hip", "attn.hip", "reader.hip")
+HEADERS = ("nsx_common.h", "raw_dot.h", "gemv_mm.h")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

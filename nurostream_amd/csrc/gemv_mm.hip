@@ -1,0 +1,621 @@
+// Fused dequant-GEMV on raw GGUF rows for 2 to 16 tokens, on gfx950's matrix
+// cores (nsx_fused_gemv; the reference's compute/triton_kernels.py:199-228
+// fuses one token).
+//
+// y = x . W^T with every weight code exact in f16 and every activation as the
+// sum of three f16 terms of a power-of-two-scaled copy: 33 significant bits,
+// so no more is lost than a product of fp32 values loses, and the matrix
+// cores' sums are fp32. v_mfma_f32_16x16x32_f16 with A = 16 rows of terms x 32
+// elements and B = 32 elements x 16 weight rows. The 16 rows of A are
+//   up to 5 tokens:  row j = term j / 5 of token j % 5, one instruction;
+//   up to 8:  row j = term j / 8 of token j % 8, then a second instruction
+//     whose rows j < 8 are term 2;
+//   up to 16: row j = token j, one instruction per term.
+// A lane holds one weight row's codes and the same row's results, so the
+// block scales multiply its own registers, without a shuffle.
+//
+// A workgroup is 8 or 16 waves; each takes its part of K and keeps its terms in
+// registers for every row it meets (a small kernel lays them out in the
+// caller's workspace: no LDS or cache traffic for activations in the loop). Per 16-row tile a wave reads its part of the
+// rows with 16-byte loads, coalesced along the rows, parks them in LDS (a
+// private buffer, so that a lane can pick up its codes at any byte offset),
+// requests the next tile's, and multiplies; the partial sums meet in LDS
+// in a fixed order, one barrier per tile. Where K exceeds what the waves hold,
+// K is taken in passes over groups of GM_GROUP tiles whose sums wait in LDS.
+//
+// Bound: the weight bytes, then the decode's VALU instructions (about 20 per 8 codes
+// of a lane). Measured, 200000 x 2880, one call: Q8_0 at 8 tokens 144 us (4.3 TB/s) against 1150
+// for the VALU kernel, which decodes a weight per 4 tokens; MXFP4 at 5 tokens 82 / 622; Q4_0 83 /
+// 626; Q4_K 98 / 645; Q6_K 157 / 494.
+#include "gemv_mm.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace {
+
+constexpr int GM_ROWS = 16;    // weight rows of a tile
+constexpr int GM_GROUP = 16;   // tiles whose sums wait in LDS between passes over K
+constexpr int GM_PS = 20;      // floats between the A rows of a partial tile (conflict-free writes)
+constexpr int GM_MAXT = 16;
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+
+// A format's K unit (the smallest part of a row with scales of its own): elements, bytes.
+template <int FMT> struct Unit { static constexpr int E = 32, B = FMT == NSX_Q8_0 ? 34 : FMT == NSX_Q4_0 ? 18 : 17; };
+template <> struct Unit<NSX_Q4_K> { static constexpr int E = 256, B = 144; };
+template <> struct Unit<NSX_Q6_K> { static constexpr int E = 256, B = 210; };
+
+// Waves of a workgroup: 16 where a sixteenth of K leaves each its 128 registers without spilling, else 8 with 256
+// (200000 x 2880: Q4_0 at 5 tokens 83 us against 99 with 8 waves, at 8 tokens 86 / 101, but at 16 tokens 150 / 106;
+// MXFP4 65536 x 4096 at 5 tokens 41 / 52; Q8_0 117 / 131, at 8 tokens 169 / 144; Q4_K and Q6_K blocks of 256 spill).
+template <int FMT>
+constexpr int gm_waves(int nm) { return Unit<FMT>::E == 32 && nm <= (FMT == NSX_Q8_0 ? 1 : 2) ? 16 : 8; }
+// Elements a wave holds terms for, in 32s: 4 registers per 32 elements and instruction, what the staged pieces leave of
+// the lane's registers (Q8_0 at 8 tokens, 65536 x 4096: 16 of them, spilling, 100 us, two passes of 8 75 us).
+template <int FMT>
+constexpr int gm_max_e32(int nm) {
+  if (gm_waves<FMT>(nm) == 16) return nm == 1 && FMT != NSX_Q8_0 ? 8 : 6;
+  if (FMT == NSX_Q8_0) return nm == 2 ? 12 : 8;
+  if (FMT == NSX_Q6_K) return nm == 1 ? 16 : 8;
+  return nm == 3 ? (FMT == NSX_Q4_K ? 8 : 12) : 16;
+}
+
+// 16-byte pieces of one row's part of a tile, which are the row's stride in LDS: not a multiple of 4, so that the 16
+// rows' reads spread over the banks.
+__host__ __device__ constexpr int gm_pieces(int bytes) {
+  const int n = (bytes + 3 + 15) / 16;
+  return n % 4 ? n : n + 1;
+}
+
+// A lane's weight row in LDS, whose first byte may sit at any offset modulo 4. Whole code words are read from the
+// aligned dwords around them and realigned in registers (a misaligned LDS word costs several aligned ones); c is the
+// word's place past the lane group's part, a constant, so that one of four addresses and shifts serves it.
+struct LdsRow {
+  const uint8_t* p;      // the row
+  const uint8_t* at[4];  // dword that holds byte k of the lane group's part of the row
+  uint32_t sh[4];        // place of that byte in it
+  __device__ __forceinline__ void set(const uint8_t* aligned, uint32_t res, uint32_t part) {
+    p = aligned + res;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      at[k] = aligned + part + ((res + k) & ~3u);
+      sh[k] = (res + k) & 3u;
+    }
+  }
+  __device__ __forceinline__ uint32_t word(int c) const {
+    const uint32_t* d = (const uint32_t*)(at[c & 3] + (c & ~3));
+    return nsx_alignbyte(d[1], d[0], sh[c & 3]);
+  }
+  __device__ __forceinline__ v2u words(int c) const {
+    const uint32_t* d = (const uint32_t*)(at[c & 3] + (c & ~3));
+    return v2u{nsx_alignbyte(d[1], d[0], sh[c & 3]), nsx_alignbyte(d[2], d[1], sh[c & 3])};
+  }
+  template <typename T>
+  __device__ __forceinline__ T get(int c) const {  // (gfx950 reads LDS at any byte offset)
+    T v;
+    __builtin_memcpy(&v, p + c, sizeof(T));
+    return v;
+  }
+};
+
+__device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
+__device__ __forceinline__ uint32_t as_u(h2 v) { return __builtin_bit_cast(uint32_t, v); }
+// two code bytes of w (selected by sel's low bytes) under 0x64: the f16 values 1024 + code
+__device__ __forceinline__ h2 biased(uint32_t w, uint32_t sel) {
+  return as_h2(__builtin_amdgcn_perm(0x64646464u, w, sel));
+}
+constexpr uint32_t SEL01 = 0x04010400u, SEL23 = 0x04030402u;
+__device__ __forceinline__ h2 both(float v) { return h2{(_Float16)v, (_Float16)v}; }
+
+template <int NM>
+__device__ __forceinline__ int gm_token(int j) { return NM == 1 ? j % 5 : NM == 2 ? j % 8 : j; }
+
+// ---------------------------------------------------------------------------
+// Activation terms, laid out as the lanes of the product kernel hold them:
+//   per unit and instruction m its operands, [piece][lane][16 B]: a format of 32-element units has one piece; Q4_K
+//   eight (sub-blocks 0..7) and one with the sub-blocks' sums / 32 (lane group 0: elements 0..7; zero elsewhere);
+//   Q6_K eight of two 16-element products each;
+//   then 16 exponents: slot j's token was scaled by 2^(its exponent).
+template <int FMT> constexpr int GM_PIECES = FMT == NSX_Q4_K ? 9 : FMT == NSX_Q6_K ? 8 : 1;
+template <int FMT>
+__host__ __device__ constexpr int64_t gm_terms_bytes(int64_t K, int nm) {
+  return K / Unit<FMT>::E * GM_PIECES<FMT> * nm * 1024;
+}
+
+// Element (of the unit) at place v (0..7) of piece pc of lane group g.
+template <int FMT>
+__device__ __forceinline__ int gm_elem(int pc, int g, int v) {
+  if constexpr (FMT == NSX_Q8_0) return 8 * g + v;
+  else if constexpr (FMT == NSX_Q4_K) return 32 * pc + 8 * g + v;
+  else if constexpr (FMT == NSX_Q4_0) return 4 * g + (v & 3) + 16 * (v >> 2);   // low nibbles, then high ones
+  else if constexpr (FMT == NSX_MXFP4) return 4 * g + (v >> 1) + 16 * (v & 1);  // a byte's low and high code side by side
+  else {  // Q6_K: products 2 pc and 2 pc + 1; product 4 (2 h + hl) + L holds elements 128 h + 32 L + 16 hl ..
+    const int pr = 2 * pc + (v >> 2), hh = pr >> 2, L = pr & 3;
+    return 128 * (hh >> 1) + 32 * L + 16 * (hh & 1) + 4 * g + (v & 3);
+  }
+}
+
+// Terms 0..2 of the scaled activation v: its leading 11 bits, the next 11, the rest; each is exact in f16 (down to
+// f16's subnormals, 2^-39 of the token's largest value). An infinite or NaN v is its own first term.
+__device__ __forceinline__ void gm_split(float v, _Float16 (&t)[3]) {
+  auto top = [](float x) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xFFFFE000u); };
+  const bool fin = fabsf(v) <= 3.4028235e38f;
+  const float hi = fin ? top(v) : v;
+  const float r = fin ? v - hi : 0.f, mid = top(r);
+  t[0] = (_Float16)hi;
+  t[1] = (_Float16)mid;
+  t[2] = (_Float16)(r - mid);
+}
+
+// Workgroup (token, part of K): the token's scale (its largest finite |x| goes to 2^14 .. 2^15) from the whole row,
+// then its slots' terms of the part's units; token 0's workgroups clear the slots that hold no token.
+template <int FMT, int NM>
+__global__ __launch_bounds__(256) void gm_terms_kernel(const void* __restrict__ x, int dt, int K, int T,
+                                                       uint8_t* __restrict__ ws) {
+  constexpr int UE = Unit<FMT>::E, PC = GM_PIECES<FMT>, ROWS = UE / 8;  // 8-element runs of a unit
+  __shared__ float part[4];
+  const int tok = blockIdx.x, tid = threadIdx.x;
+  const int64_t x0 = (int64_t)tok * K;
+  float mx = 0.f;
+  for (int k = tid; k < K; k += 256 * 8) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = nsx_load_act(x, dt, x0 + min(k + 256 * i, K - 1));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mx = fabsf(v[i]) <= 3.4028235e38f ? fmaxf(mx, fabsf(v[i])) : mx;
+  }
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if ((tid & 63) == 0) part[tid >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  int ex = 15;
+  if (mx > 0.f) (void)frexpf(mx, &ex);  // mx < 2^ex
+  const int e = 15 - ex;
+  int32_t* exps = (int32_t*)(ws + gm_terms_bytes<FMT>(K, NM));
+  auto store = [&](int slot, int m, int u, int pc, int g, const h8& h) {
+    *(h8*)(ws + ((((int64_t)u * PC + pc) * NM + m) * 64 + 16 * g + slot) * 16) = h;
+  };
+  // run r of 8 elements -> piece pc = r / 4 of lane group g = r % 4 (Q4_K's sums: below)
+  const int runs = K / 8, per = (runs + (int)gridDim.y - 1) / (int)gridDim.y;
+  const int r1 = min(runs, per * ((int)blockIdx.y + 1));
+  for (int r = per * (int)blockIdx.y + tid; r < r1; r += 256) {
+    const int u = r / ROWS, pc = (r % ROWS) >> 2, g = r & 3;
+    _Float16 t[8][3];
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+      gm_split(ldexpf(nsx_load_act(x, dt, x0 + (int64_t)u * UE + gm_elem<FMT>(pc, g, v)), e), t[v]);
+#pragma unroll
+    for (int term = 0; term < 3; ++term) {
+      h8 h;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) h[v] = t[v][term];
+      if (NM == 1) store(5 * term + tok, 0, u, pc, g, h);
+      else if (NM == 2) store(term == 1 ? 8 + tok : tok, term == 2 ? 1 : 0, u, pc, g, h);
+      else store(tok, term, u, pc, g, h);
+    }
+  }
+  if constexpr (FMT == NSX_Q4_K) {  // one thread per super-block of this workgroup's part
+    const int all = K / UE, pu = (all + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int u = pu * (int)blockIdx.y + (tid >> 3);  // 8 threads per unit, one sub-block each
+    const bool on = (tid >> 3) < pu && u < all;
+    float s = 0.f;
+    for (int i = 0; i < 32; ++i) s += on ? ldexpf(nsx_load_act(x, dt, x0 + (int64_t)u * UE + 32 * (tid & 7) + i), e) : 0.f;
+    _Float16 t[3];
+    gm_split(s * 0.03125f, t);  // (32 values below 2^15: within f16's range)
+    if (on) {
+#pragma unroll
+      for (int term = 0; term < 3; ++term) {
+        const int slot = NM == 1 ? 5 * term + tok : NM == 2 ? (term == 1 ? 8 + tok : tok) : tok;
+        const int m = NM == 1 ? 0 : NM == 2 ? (term == 2 ? 1 : 0) : term;
+        uint8_t* p = ws + ((((int64_t)u * PC + 8) * NM + m) * 64 + slot) * 16;
+        *(_Float16*)(p + 2 * (tid & 7)) = t[term];
+        for (int g = 1; g < 4; ++g) *(_Float16*)(p + 16 * 16 * g + 2 * (tid & 7)) = (_Float16)0.f;
+      }
+    }
+  }
+  if (blockIdx.y == 0 && tid < 16 && gm_token<NM>(tid) == tok) exps[tid] = e;
+  if (tok == 0) {  // slots without a token (NM 2: the second instruction has 8 more)
+    const int all = K / UE * PC;
+    for (int i = (int)blockIdx.y * 256 + tid; i < all * NM * 64; i += 256 * (int)gridDim.y) {
+      const int slot = i & 15, m = (i >> 6) % NM;
+      const bool none = gm_token<NM>(slot) >= T || (NM == 1 && slot == 15) || (NM == 2 && m == 1 && slot >= 8);
+      if (none) *(v4u*)(ws + (int64_t)i * 16) = v4u{0, 0, 0, 0};
+    }
+    if (blockIdx.y == 0 && tid < 16 && gm_token<NM>(tid) >= T) exps[tid] = 0;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// the products
+
+struct GmArgs {
+  const uint8_t* base;
+  uint32_t head, range;
+  int n_rows, K, T;
+  const uint8_t* terms;
+  float* y;
+  int64_t ystride;
+  const float* bias;
+  const float* resid;  // may be y
+  int npass, units;    // passes over K, units of a full pass
+  int part_bytes;      // LDS bytes of a wave's part of a tile (GM_ROWS rows)
+};
+
+// The terms of one unit in registers.
+template <int FMT, int NM>
+struct Terms {
+  h8 a[GM_PIECES<FMT>][NM];
+};
+
+__device__ __forceinline__ h8 gm_h8(h2 a, h2 b, h2 c, h2 d) {
+  return __builtin_bit_cast(h8, v4u{as_u(a), as_u(b), as_u(c), as_u(d)});
+}
+
+template <int N>
+__device__ __forceinline__ v4f gm_mfma(const h8 (&x)[N], h8 w, v4f c) {
+#pragma unroll
+  for (int m = 0; m < N; ++m) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[m], w, c, 0, 0, 0);
+  return c;
+}
+
+// y += unit (its bytes from o on in this lane's weight row) times the terms. MXFP4: times the tokens' scales as well (te, the
+// A rows' scale exponents): a block scale alone may lie far outside the range of the product. The other formats' scales
+// are f16, so the sums cannot leave fp32's range and the tokens' scales wait for the end.
+template <int FMT, int NM>
+__device__ __forceinline__ void gm_unit(const LdsRow& R, const LdsRow& S0, int o, const Terms<FMT, NM>& X, int g, const int (&te)[4], v4f& y) {
+  const v4f zero = {0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const v4f& d, float s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = fmaf(FMT == NSX_MXFP4 ? __builtin_amdgcn_ldexpf(d[i], -te[i]) : d[i], s, y[i]);
+  };
+  if constexpr (FMT == NSX_Q8_0) {
+    const v2u w = R.words(o + 2);
+    const h2 off = both(-1152.f);
+    const uint32_t w0 = w.x ^ 0x80808080u, w1 = w.y ^ 0x80808080u;
+    const h8 b = gm_h8(biased(w0, SEL01) + off, biased(w0, SEL23) + off, biased(w1, SEL01) + off, biased(w1, SEL23) + off);
+    add(gm_mfma(X.a[0], b, zero), nsx_h2f(R.get<uint16_t>(o)));
+  } else if constexpr (FMT == NSX_Q4_0) {
+    const uint32_t w = R.word(o + 2), lo = w & 0x0F0F0F0Fu, hi = w & 0xF0F0F0F0u;
+    const h2 off = both(-1032.f), s16 = both(0.0625f), off16 = both(-72.f);
+    const h8 b = gm_h8(biased(lo, SEL01) + off, biased(lo, SEL23) + off,
+                       __builtin_elementwise_fma(biased(hi, SEL01), s16, off16),
+                       __builtin_elementwise_fma(biased(hi, SEL23), s16, off16));
+    add(gm_mfma(X.a[0], b, zero), nsx_h2f(R.get<uint16_t>(o)));
+  } else if constexpr (FMT == NSX_MXFP4) {
+    const uint32_t w = R.word(o + 1);
+    const h8 b = gm_h8(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 1),
+                       __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 3));
+    add(gm_mfma(X.a[0], b, zero), nsx_mx_scale_half(R.get<uint8_t>(o)));
+  } else if constexpr (FMT == NSX_Q4_K) {
+    const v4u H = R.get<v4u>(o);  // d | dmin, scales[12]
+    const uint32_t sc03 = H.y & 0x3F3F3F3Fu, sc47 = (H.w & 0x0F0F0F0Fu) | ((H.y >> 2) & 0x30303030u);
+    const uint32_t mn03 = H.z & 0x3F3F3F3Fu, mn47 = ((H.w >> 4) & 0x0F0F0F0Fu) | ((H.z >> 2) & 0x30303030u);
+    const h2 k1024 = both(1024.f), km1024 = both(-1024.f), s16 = both(0.0625f), km64 = both(-64.f);
+    v4f acc = zero;
+#pragma unroll
+    for (int pr = 0; pr < 4; ++pr) {  // sub-blocks 2 pr (low nibbles) and 2 pr + 1 (high ones)
+      const uint32_t scw = pr < 2 ? sc03 : sc47, b0 = 2u * (pr & 1);
+      const h2 ml = biased(scw, 0x04000400u | b0 << 16 | b0) - k1024;  // (sc, sc)
+      const h2 mh = __builtin_elementwise_fma(biased(scw, 0x04000400u | (b0 + 1) << 16 | (b0 + 1)), s16, km64);
+      const h2 cl = ml * km1024, ch = mh * km1024;
+      const v2u w = R.get<v2u>(o + 16 + 32 * pr + 8 * g);  // (rows of 16-byte pieces, 4-byte aligned: aligned here)
+      const uint32_t l0 = w.x & 0x0F0F0F0Fu, l1 = w.y & 0x0F0F0F0Fu, h0 = w.x & 0xF0F0F0F0u, h1 = w.y & 0xF0F0F0F0u;
+      auto sq = [](uint32_t q, uint32_t sel, h2 m, h2 c) { return __builtin_elementwise_fma(biased(q, sel), m, c); };
+      acc = gm_mfma(X.a[2 * pr], gm_h8(sq(l0, SEL01, ml, cl), sq(l0, SEL23, ml, cl), sq(l1, SEL01, ml, cl), sq(l1, SEL23, ml, cl)), acc);
+      acc = gm_mfma(X.a[2 * pr + 1], gm_h8(sq(h0, SEL01, mh, ch), sq(h0, SEL23, mh, ch), sq(h1, SEL01, mh, ch), sq(h1, SEL23, mh, ch)), acc);
+    }
+    const h8 mins = gm_h8(biased(mn03, SEL01) - k1024, biased(mn03, SEL23) - k1024, biased(mn47, SEL01) - k1024,
+                          biased(mn47, SEL23) - k1024);
+    const v4f am = gm_mfma(X.a[8], mins, zero);
+    add(acc, nsx_h2f(H.x & 0xFFFFu));
+    add(am, -32.f * nsx_h2f(H.x >> 16));
+  } else {  // Q6_K: a scale for every 16 elements, sc (q - 32) takes more than f16's 11 bits: 16-element products
+    v4f acc = zero;
+    const h2 off = both(-1056.f);
+    uint32_t scw[4];  // the 16 scales
+#pragma unroll
+    for (int i = 0; i < 4; ++i) scw[i] = S0.word(o + 192 + 4 * i);
+#pragma unroll
+    for (int hh = 0; hh < 4; ++hh) {
+      const int h = hh >> 1, hl = hh & 1;
+      const uint32_t qa = R.word(o + 64 * h + 16 * hl), qb = R.word(o + 64 * h + 32 + 16 * hl);
+      const uint32_t qh = R.word(o + 128 + 32 * h + 16 * hl);
+#pragma unroll
+      for (int L = 0; L < 4; ++L) {
+        const uint32_t nib = ((L & 1 ? qb : qa) >> (4 * (L >> 1))) & 0x0F0F0F0Fu;
+        const uint32_t top = L == 0 ? qh << 4 : L == 1 ? qh << 2 : L == 2 ? qh : qh >> 2;
+        const uint32_t q = nib | (top & 0x30303030u);
+        const v2u bw = {as_u(biased(q, SEL01) + off), as_u(biased(q, SEL23) + off)};
+        const h4 b = __builtin_bit_cast(h4, bw);
+        v4f d = zero;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+          const h8 x = X.a[2 * hh + (L >> 1)][m];
+          const h4 xa = L & 1 ? h4{x[4], x[5], x[6], x[7]} : h4{x[0], x[1], x[2], x[3]};
+          d = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, b, d, 0, 0, 0);
+        }
+        const int si = 8 * h + hl + 2 * L;
+        const float sc = (float)(int8_t)(scw[si >> 2] >> (8 * (si & 3)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = fmaf(sc, d[i], acc[i]);
+      }
+    }
+    add(acc, nsx_h2f(R.get<uint16_t>(o + 208)));
+  }
+}
+
+__device__ __forceinline__ void gm_barrier() {  // LDS only: the next tile's loads stay in flight
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int FMT, int NM, int MAXU>
+__global__ __launch_bounds__(64 * gm_waves<FMT>(NM)) void gemv_mm_kernel(GmArgs a) {
+  constexpr int UE = Unit<FMT>::E, UB = Unit<FMT>::B, W = gm_waves<FMT>(NM);
+  constexpr int LOADS = (GM_ROWS * gm_pieces(MAXU * UB) + 63) / 64;  // 16-byte loads of a tile per lane
+  extern __shared__ __align__(16) uint8_t gm_smem[];
+  const int lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, g = lane >> 4;
+  uint8_t* buf = gm_smem + wave * a.part_bytes;
+  constexpr int PART = GM_ROWS * GM_PS;
+  float* parts = (float*)(gm_smem + W * a.part_bytes);  // [2][wave][A row][GM_PS]
+  float* sums = parts + 2 * W * PART;                             // npass > 1: [tile of the group][16 token + row]
+  const __amdgpu_buffer_rsrc_t rs = nsx_rsrc(a.base, a.range);
+  const uint32_t rb = (uint32_t)(a.K / UE) * UB;
+  const int ntiles = (a.n_rows + GM_ROWS - 1) / GM_ROWS;
+  const int mine = (ntiles - 1 - (int)blockIdx.x) / (int)gridDim.x + 1;  // (the grid is at most ntiles)
+
+  // This wave's part of a pass: units own0 .. own0 + own - 1, read as the MAXU units from u0 on (the neighbours' among
+  // them have zero terms here), so that every place in LDS is a constant.
+  constexpr int N16 = gm_pieces(MAXU * UB), PIECES = GM_ROWS * N16;
+  int u0 = 0, own0 = 0, own = 0;
+  LdsRow row, row0p;             // this lane's weight row in LDS, from its lane group's codes on; from its start
+  uint32_t goff[LOADS];          // a tile's pieces: byte offset of piece lane + 64 q (in LDS at 16 (lane + 64 q))
+  v4u stage[LOADS];
+  Terms<FMT, NM> X[MAXU];
+  int te[4];  // scale exponents of A rows 4 g .. 4 g + 3
+
+  // Piece p of a tile: row p / N16 (at most rlast), bytes 16 (p % N16) .. from the dword that holds the first byte of
+  // the wave's part of the row. The last pieces run into the next row. Lanes past the last piece repeat it.
+  auto piece = [&](int q, int rlast) {
+    const int p = min(lane + 64 * q, PIECES - 1), r = p / N16, c = p - r * N16;
+    return ((a.head + (uint32_t)min(r, rlast) * rb + (uint32_t)u0 * UB) & ~3u) + (uint32_t)c * 16u;
+  };
+  auto slot = [&](int q) { return min(lane + 64 * q, PIECES - 1); };
+  auto set_pass = [&](int pass) {
+    const int all = a.K / UE, p0 = pass * a.units, pn = min(a.units, all - p0);
+    const int per = pn / W, extra = pn % W;
+    own = per + (wave < extra ? 1 : 0);
+    own0 = p0 + wave * per + min(wave, extra);
+    u0 = min(own0, all - MAXU);
+    const uint32_t res = (a.head + (uint32_t)c16 * rb + (uint32_t)u0 * UB) & 3u;
+    row.set(buf + c16 * N16 * 16, res, (FMT == NSX_Q8_0 ? 8u : 4u) * (uint32_t)g);
+    row0p.set(buf + c16 * N16 * 16, res, 0);
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) goff[q] = piece(q, GM_ROWS - 1);
+  };
+  // A tile whose pieces could cross the end of the matrix (the last one): rows past it read its last row (their
+  // results are not stored), and a piece that would cross it is moved back to end there, in LDS as well.
+  const uint32_t rend = (a.range + 3u) & ~3u;
+  auto row0 = [&](int i) { return ((int)blockIdx.x + i * (int)gridDim.x) * GM_ROWS; };
+  auto at_end = [&](int i) { return (int64_t)(row0(i) + GM_ROWS) * rb + a.head + 64 > (int64_t)a.range; };
+  auto rows_left = [&](int i) {  // (opaque: this rare case's places are not worth registers in the loop)
+    int n = a.n_rows - 1 - row0(i);
+    asm volatile("" : "+s"(n));
+    return n;
+  };
+  // The loads of tile i (tiles start a multiple of 4 bytes apart: the pieces' places are the same in every tile).
+  auto issue = [&](int i) {
+    const uint32_t so = (uint32_t)row0(i) * rb;
+    if (!at_end(i)) {
+#pragma unroll
+      for (int q = 0; q < LOADS; ++q)
+        stage[q] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rs, goff[q], so, 0));
+    } else {
+      const int n = rows_left(i);
+#pragma unroll
+      for (int q = 0; q < LOADS; ++q)
+        stage[q] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rs, min(piece(q, n) + so, rend - 16u), 0, 0));
+    }
+  };
+  auto park = [&](int i) {  // the loaded pieces into LDS
+    if (!at_end(i)) {
+#pragma unroll
+      for (int q = 0; q < LOADS; ++q) *(v4u*)(buf + 16 * slot(q)) = stage[q];
+    } else {
+      const int n = rows_left(i);
+#pragma unroll
+      for (int q = 0; q < LOADS; ++q) {
+        const uint32_t at = piece(q, n) + (uint32_t)row0(i) * rb;
+        __builtin_memcpy(buf + 16 * slot(q) - (at - min(at, rend - 16u)), &stage[q], 16);
+      }
+    }
+  };
+  // The terms of the pass (those of the neighbours' units zero).
+  auto take_terms = [&]() {
+    const v4u zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < MAXU; ++u) {
+      const bool mine = (uint32_t)(u0 + u - own0) < (uint32_t)own;
+#pragma unroll
+      for (int pc = 0; pc < GM_PIECES<FMT>; ++pc)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+          const v4u t = *(const v4u*)(a.terms + ((((int64_t)(u0 + u) * GM_PIECES<FMT> + pc) * NM + m) * 64 + lane) * 16);
+          X[u].a[pc][m] = __builtin_bit_cast(h8, mine ? t : zero);
+        }
+    }
+  };
+  const int32_t* exps = (const int32_t*)(a.terms + gm_terms_bytes<FMT>(a.K, NM));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) te[i] = exps[4 * g + i];
+
+  int flip = 0;
+  for (int i0 = 0; i0 < mine; i0 += a.npass > 1 ? GM_GROUP : mine) {
+    const int i1 = a.npass > 1 ? min(mine, i0 + GM_GROUP) : mine;
+    for (int pass = 0; pass < a.npass; ++pass) {
+      if (a.npass > 1 || i0 == 0) {
+        set_pass(pass);
+        issue(i0);
+        take_terms();
+      }
+      // the sums of tile i (the waves' partials are in buffer `flip`)
+      auto finish = [&](int i) {
+        if ((int)threadIdx.x >= GM_ROWS * a.T) return;
+        const int tok = threadIdx.x >> 4, r = threadIdx.x & 15, at = row0(i) + r;
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+          const float* pw = parts + (flip * W + w) * PART + tok * GM_PS + r;
+          v += NM == 1 ? (pw[0] + pw[5 * GM_PS]) + pw[10 * GM_PS] : NM == 2 ? pw[0] + pw[8 * GM_PS] : pw[0];
+        }
+        if (pass > 0) v += sums[(i - i0) * 256 + threadIdx.x];
+        if (pass + 1 < a.npass) {
+          sums[(i - i0) * 256 + threadIdx.x] = v;
+        } else if (at < a.n_rows) {  // the reference's order: resid + (x @ W.T + bias)
+          const int64_t o = (int64_t)tok * a.ystride + at;
+          if (a.bias) v += a.bias[at];
+          if (a.resid) v = a.resid[o] + v;
+          a.y[o] = v;
+        }
+      };
+      for (int i = i0; i < i1; ++i) {
+        v4f y = {0.f, 0.f, 0.f, 0.f};
+        park(i);
+        if (i + 1 < i1) issue(i + 1);
+        asm volatile("" ::: "memory");  // the wave's LDS operations run in order
+        if (i > i0) {  // the tile before, behind this one's requests
+          finish(i - 1);
+          flip ^= 1;
+        }
+#pragma unroll
+        for (int u = 0; u < MAXU; ++u) gm_unit<FMT, NM>(row, row0p, u * UB, X[u], g, te, y);
+        // (the buffer that every wave has read by the barrier it met after the tile before)
+        float* part = parts + (flip * W + wave) * PART;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[(4 * g + r) * GM_PS + c16] = FMT == NSX_MXFP4 ? y[r] : __builtin_amdgcn_ldexpf(y[r], -te[r]);
+        gm_barrier();
+      }
+      finish(i1 - 1);
+      flip ^= 1;
+    }
+  }
+}
+
+template <int FMT, int NM, int E32>
+int gm_launch(GmArgs a, hipStream_t st) {
+  constexpr int MAXU = E32 * 32 / Unit<FMT>::E;
+  a.part_bytes = GM_ROWS * gm_pieces(MAXU * Unit<FMT>::B) * 16;
+  constexpr int W = gm_waves<FMT>(NM);
+  const size_t lds = (size_t)W * a.part_bytes + 2 * W * GM_ROWS * GM_PS * sizeof(float) +
+                     (a.npass > 1 ? GM_GROUP * 256 * sizeof(float) : 0);
+  const void* k = (const void*)gemv_mm_kernel<FMT, NM, MAXU>;
+  if (lds > 64 * 1024) NSX_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const int64_t grid = std::min<int64_t>(nsx_cdiv(a.n_rows, GM_ROWS), nsx_resident_workgroups(k, lds, 64 * W));
+  hipLaunchKernelGGL((gemv_mm_kernel<FMT, NM, MAXU>), dim3((unsigned)grid), dim3(64 * W), lds, st, a);
+  NSX_LAUNCHED();
+  return NSX_OK;
+}
+
+// K in as few passes as the waves can hold, of equal length; the smallest kernel that holds one.
+template <int FMT, int NM>
+int gm_size(GmArgs a, hipStream_t st) {
+  constexpr int UE = Unit<FMT>::E, CAP = gm_max_e32<FMT>(NM);
+  const int all = a.K / UE;
+  a.npass = (int)nsx_cdiv(all, gm_waves<FMT>(NM) * CAP * 32 / UE);
+  a.units = (int)nsx_cdiv(all, a.npass);
+  const int e32 = (int)nsx_cdiv(a.units, gm_waves<FMT>(NM)) * (UE / 32);
+  if constexpr (UE == 32) {
+    if (e32 <= 4) return gm_launch<FMT, NM, 4>(a, st);
+    if (e32 <= 6) return gm_launch<FMT, NM, 6>(a, st);
+  }
+  if constexpr (CAP >= 8) {
+    if (e32 <= 8) return gm_launch<FMT, NM, 8>(a, st);
+  }
+  if constexpr (UE == 32 && CAP >= 12) {
+    if (e32 <= 12) return gm_launch<FMT, NM, 12>(a, st);
+  }
+  if constexpr (CAP >= 16) return gm_launch<FMT, NM, 16>(a, st);
+  return nsx_fail(NSX_EINVAL, "K %d", a.K);
+}
+
+template <int FMT, int NM>
+int gm_run(const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtype, int64_t T, float* y, const float* bias,
+           const float* resid, uint8_t* ws, hipStream_t st) {
+  // the terms, in as many parts as keep a thread's share small
+  const unsigned parts = (unsigned)std::max<int64_t>(1, std::min<int64_t>(16, nsx_cdiv(K, 2048)));
+  hipLaunchKernelGGL((gm_terms_kernel<FMT, NM>), dim3((unsigned)T, parts), dim3(256), 0, st, x, x_dtype, (int)K, (int)T, ws);
+  NSX_LAUNCHED();
+  const int64_t rb = K / Unit<FMT>::E * Unit<FMT>::B;
+  const int64_t per = std::max<int64_t>(1, ((int64_t)1 << 31) / rb / GM_ROWS) * GM_ROWS;  // 32-bit byte offsets
+  for (int64_t r0 = 0; r0 < n_rows; r0 += per) {
+    const int64_t nr = std::min(per, n_rows - r0);
+    const uint8_t* p = (const uint8_t*)raw + r0 * rb;
+    const uintptr_t at = (uintptr_t)p & ~(uintptr_t)3;
+    GmArgs a{};
+    a.base = (const uint8_t*)at;
+    a.head = (uint32_t)((uintptr_t)p - at);
+    a.range = a.head + (uint32_t)(nr * rb);
+    a.n_rows = (int)nr;
+    a.K = (int)K;
+    a.T = (int)T;
+    a.terms = ws;
+    a.y = y + r0;
+    a.ystride = n_rows;
+    a.bias = bias ? bias + r0 : nullptr;
+    a.resid = resid ? resid + r0 : nullptr;
+    if (int rc = gm_size<FMT, NM>(a, st)) return rc;
+  }
+  return NSX_OK;
+}
+
+int gm_mode(int64_t T) { return T <= 5 ? 1 : T <= 8 ? 2 : 3; }  // instructions per 32 elements
+
+template <int FMT>
+int gm_fmt(const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtype, int64_t T, float* y, const float* bias,
+           const float* resid, uint8_t* ws, hipStream_t st) {
+  switch (gm_mode(T)) {
+    case 1: return gm_run<FMT, 1>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, ws, st);
+    case 2: return gm_run<FMT, 2>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, ws, st);
+    default: return gm_run<FMT, 3>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, ws, st);
+  }
+}
+
+}  // namespace
+
+int64_t nsx_gemv_mm_workspace(int t, int64_t n_rows, int64_t K, int64_t T) {
+  if (T < 2 || T > GM_MAXT || K < 128) return 0;  // (a wave reads at least 4 blocks of 32)
+  // below these sizes the VALU kernel's one launch is the shorter one (us, VALU / here: Q4_0 at 2 tokens 2880 x 2880
+  // 10.3 / 11.0, 5120 x 2880 13.7 / 12.7; at 3 512 x 4096 12.3 / 12.3, 2048 x 4096 17.1 / 11.7; at 5 512 x 4096 18.4 /
+  // 11.5; Q8_0 and MXFP4 cross there too. The K-quants' wider blocks: Q4_K at 2 tokens 5120 x 2816 13.8 / 16.7,
+  // 12288 x 4096 31.8 / 20.9; Q6_K 23.3 / 26.7, 65536 x 4096 91 / 66; at 3 5120 x 2816 16.8 / 20.4, 12288 x 4096 35 / 27)
+  const int64_t least = T == 2 ? (t == NSX_Q6_K ? 64ll : t == NSX_Q4_K ? 24ll : 12ll)
+                      : T <= 4 ? (t == NSX_Q6_K ? 24ll : 4ll) : 1ll;
+  if (n_rows * K < least << 20) return 0;
+  int64_t b = 0;
+  switch (t) {
+    case NSX_MXFP4: b = gm_terms_bytes<NSX_MXFP4>(K, gm_mode(T)); break;
+    case NSX_Q4_0: b = gm_terms_bytes<NSX_Q4_0>(K, gm_mode(T)); break;
+    case NSX_Q8_0: b = gm_terms_bytes<NSX_Q8_0>(K, gm_mode(T)); break;
+    case NSX_Q4_K: b = gm_terms_bytes<NSX_Q4_K>(K, gm_mode(T)); break;
+    case NSX_Q6_K: b = gm_terms_bytes<NSX_Q6_K>(K, gm_mode(T)); break;
+    default: return 0;
+  }
+  return b + 64;
+}
+
+int nsx_gemv_mm(int t, const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtype, int64_t T, float* y,
+                const float* bias, const float* resid, void* ws, hipStream_t st) {
+  uint8_t* w = (uint8_t*)ws;
+  switch (t) {
+    case NSX_MXFP4: return gm_fmt<NSX_MXFP4>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, w, st);
+    case NSX_Q4_0: return gm_fmt<NSX_Q4_0>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, w, st);
+    case NSX_Q8_0: return gm_fmt<NSX_Q8_0>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, w, st);
+    case NSX_Q4_K: return gm_fmt<NSX_Q4_K>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, w, st);
+    case NSX_Q6_K: return gm_fmt<NSX_Q6_K>(raw, n_rows, K, x, x_dtype, T, y, bias, resid, w, st);
+  }
+  return nsx_fail(NSX_ENOTIMPL, "ggml type %d", t);
+}

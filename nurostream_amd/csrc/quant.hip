@@ -7,6 +7,7 @@
 #include "nsx_common.h"
 #include "mx.h"
 #include "raw_dot.h"
+#include "gemv_mm.h"
 
 #include <algorithm>
 #include <mutex>
@@ -776,6 +777,18 @@ extern "C" int nsx_fused_gemv(int t, const void* raw, int64_t n_rows, int64_t K,
 extern "C" int nsx_fused_gemv_ex(int t, const void* raw, int64_t n_rows, int64_t K, const void* x,
                                  int x_dtype, int64_t T, float* y, const float* bias, const float* resid,
                                  void* stream) {
+  return nsx_fused_gemv_ws(t, raw, n_rows, K, x, x_dtype, T, y, bias, resid, nullptr, 0, stream);
+}
+
+extern "C" int64_t nsx_gemv_workspace_bytes(int t, int64_t n_rows, int64_t K, int64_t T) {
+  const int BE = nsx_block_elems(t);
+  if (BE <= 0 || n_rows <= 0 || K <= 0 || K % BE != 0) return 0;
+  return nsx_gemv_mm_workspace(t, n_rows, K, T);
+}
+
+extern "C" int nsx_fused_gemv_ws(int t, const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtype,
+                                 int64_t T, float* y, const float* bias, const float* resid, void* workspace,
+                                 int64_t workspace_bytes, void* stream) {
   const int BE = nsx_block_elems(t), BB = nsx_block_bytes(t);
   NSX_REQUIRE(BB > 0, NSX_ENOTIMPL, "no fused kernel for ggml type %d", t);
   NSX_REQUIRE(n_rows >= 0 && K > 0 && K % BE == 0, NSX_EINVAL,
@@ -790,6 +803,12 @@ extern "C" int nsx_fused_gemv_ex(int t, const void* raw, int64_t n_rows, int64_t
   if (t == NSX_Q4_K)
     NSX_REQUIRE(((uintptr_t)raw & 3) == 0, NSX_EINVAL, "Q4_K rows must be 4-byte aligned");
   hipStream_t st = S(stream);
+  if (workspace) {
+    const int64_t need = nsx_gemv_mm_workspace(t, n_rows, K, T);
+    NSX_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0, NSX_EINVAL,
+                "workspace of %lld bytes, need %lld, 16-byte aligned", (long long)workspace_bytes, (long long)need);
+    if (need > 0) return nsx_gemv_mm(t, raw, n_rows, K, x, x_dtype, T, y, bias, resid, workspace, st);
+  }
   // tokens per launch: as many as one workgroup's LDS holds (<= 64 KiB staged)
   int64_t chunk = 16;
   while (chunk > 1 && chunk * (K + K / 32) * 4 > 64 * 1024) chunk /= 2;

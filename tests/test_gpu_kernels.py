@@ -183,6 +183,56 @@ def test_fused_gemv_bias_residual_epilogue(dev, fmt, T, rows, K):
         fused_gemv(raw_t, t, xt, rows, K, out_dtype=torch.float32, bias=bt[:-1])
 
 
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "MXFP4", "Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T,rows,K,offset,xdt", [
+    (2, 9001, 8192, 0, torch.float32), (5, 401, 2816, 1, torch.float32), (6, 263, 4096, 2, torch.float16),
+    (8, 1055, 1024, 3, torch.float32), (9, 300, 5120, 0, torch.bfloat16), (16, 400, 2816, 1, torch.float32),
+    (16, 129, 15872, 0, torch.float32), (16, 8193, 256, 2, torch.float32), (5, 9001, 256, 3, torch.float32)])
+def test_fused_gemv_matrix_core_path(dev, fmt, T, rows, K, offset, xdt):
+    """Several tokens on the matrix cores: a last tile of 1 to 16 rows, rows at any byte, every arrangement of the
+    terms (up to 5, 8, 16 tokens), K in one pass and in several (over more than one group of tiles), each activation
+    type, activations from 1e-6 to 1e3. The weight codes and three terms of each activation are exact, so what is left
+    is the rounding of K fp32 sums: in practice sqrt(K) 2^-24 of a row's size, 1e-5 at most."""
+    from nurostream_amd import _native as N
+    from nurostream_amd.compute.kernels import fused_gemv
+    from nurostream_amd.compute.quant import dequantize
+    t = getattr(OQ, fmt)
+    offset = offset if fmt != "Q4_K" else 0  # (Q4_K rows are 4-byte aligned)
+    assert N.load().nsx_gemv_workspace_bytes(t, rows, K, T) > 0
+    raw = torch.from_numpy(_gemv_case(fmt, rows, K, seed=rows + T))
+    buf = torch.zeros(raw.numel() + offset, dtype=torch.uint8, device=dev)
+    w = buf[offset:]
+    w.copy_(raw)
+    g = torch.Generator().manual_seed(K + T)
+    x = torch.randn(T, K, generator=g) * torch.exp(torch.empty(T, K).uniform_(-14, 7, generator=g))
+    x[T - 1] *= 1e-30 if xdt == torch.float32 else 1  # a token far smaller than the others
+    x = x.to(xdt).to(dev)
+    W = dequantize(w, t, rows * K, torch.float32).reshape(rows, K).double()
+    # (no library product: its workspace would stay in a segment of W's size)
+    ref = torch.stack([(W * x[i].double()).sum(1) for i in range(T)]).cpu().numpy()
+    del W
+    torch.cuda.empty_cache()  # (later tests look at fresh device allocations)
+    b, r = torch.randn(rows, generator=g).to(dev), torch.randn(T, rows, generator=g).to(dev)
+    y = fused_gemv(w, t, x, rows, K, out_dtype=torch.float32)
+    for i in range(T):
+        assert rel_max(to_np(y[i]), ref[i]) < 1e-5, i
+    yb = fused_gemv(w, t, x, rows, K, out_dtype=torch.float32, bias=b, resid=r)
+    torch.testing.assert_close(yb, r + (y + b), rtol=0, atol=0)
+    ws = torch.empty(N.load().nsx_gemv_workspace_bytes(t, rows, K, T), dtype=torch.uint8, device=dev)
+    out = r.clone()  # the residual in place
+    N.check(N.load().nsx_fused_gemv_ws(t, w.data_ptr(), rows, K, x.data_ptr(), N.act_dtype_code(xdt), T, out.data_ptr(),
+                                       b.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), N.stream_ptr(dev)), "ws")
+    assert torch.equal(out, yb)
+    with pytest.raises(ValueError):  # a workspace too small
+        N.check(N.load().nsx_fused_gemv_ws(t, w.data_ptr(), rows, K, x.data_ptr(), N.act_dtype_code(xdt), T,
+                                           out.data_ptr(), None, None, ws.data_ptr(), ws.numel() - 1,
+                                           N.stream_ptr(dev)), "ws")
+    x[0, 3], x[1, 5] = float("inf"), float("nan")  # only their own tokens' outputs turn non-finite
+    z = fused_gemv(w, t, x, rows, K, out_dtype=torch.float32)
+    assert bool(torch.isnan(z[1]).all()) and not bool(torch.isfinite(z[0]).all())
+    assert torch.equal(z[2:], y[2:])
+
+
 @pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
 def test_fused_gemv_half_activations(dev, xdt):
     from nurostream_amd.compute.kernels import fused_gemv
