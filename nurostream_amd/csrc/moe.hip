@@ -1415,8 +1415,8 @@ constexpr int GRP_GU_T = 64;         // tokens per MXFP4 gate/up work item (GRP_
 // the resident workgroups (the 36-layer GPT-OSS stack at T = 8, at most 1485 units on 512 workgroups: 23.7 us per
 // layer one workgroup per unit, 25.8 persistent; config 3, T = 128: 89.7 -> 84.5 us persistent)
 constexpr int GRP_DN_PERSIST = 8;
-constexpr int GRP_MAX_PAIRS = 4096;  // pairs per sort (nsx_moe_forward splits larger T)
-constexpr int GRP_CHUNKS = GRP_MAX_PAIRS / 64;
+constexpr int GRP_MAX_PAIRS = 8192;  // pairs per sort (nsx_moe_forward splits larger T)
+constexpr int GRP_SORT_SMALL = 4096;  // up to this many the sort kernel with half the LDS and loads
 
 __host__ __device__ __forceinline__ int grp_max_items(int E, int P, int tpi = GRP_TPI) {
   return (E < P ? E : P) + (P + tpi - 1) / tpi;
@@ -1472,15 +1472,16 @@ __device__ __forceinline__ uint64_t grp_match(bool valid, int e) {
 // One workgroup, after the router phase's top-k: a stable counting sort of
 // the pairs by expert (64-pair chunks, per-chunk counts, prefix over chunks),
 // the work items and the per-token combine order.
+template <int MAXP>  // P <= MAXP
 __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeDev a) {
-  __shared__ uint16_t s_run[GRP_CHUNKS][MAX_EXPERTS];  // chunk counts, then exclusive prefix over chunks
+  __shared__ uint16_t s_run[MAXP / 64][MAX_EXPERTS];  // chunk counts, then exclusive prefix over chunks
   __shared__ int s_cnt[MAX_EXPERTS], s_off[MAX_EXPERTS];
-  __shared__ int s_pc[2][MAX_EXPERTS + GRP_MAX_PAIRS / GRP_GU_T + 1];  // cost prefixes of the gate/up items: gate/up, down
-  __shared__ uint8_t s_exp[GRP_MAX_PAIRS];
+  __shared__ int s_pc[2][MAX_EXPERTS + MAXP / GRP_GU_T + 1];  // cost prefixes of the gate/up items: gate/up, down
+  __shared__ uint8_t s_exp[MAXP];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = __lane_id();
   const int T = a.T, k = a.top_k, E = a.E, P = T * k;
   const int nch = (P + 63) / 64;
-  for (int i = tid; i < GRP_CHUNKS * MAX_EXPERTS; i += 1024) (&s_run[0][0])[i] = 0;
+  for (int i = tid; i < MAXP / 64 * MAX_EXPERTS; i += 1024) (&s_run[0][0])[i] = 0;
   if (a.topk_in_sort) {  // (T < 16: a wave per token) the top-k from the router's logits, as topk_kernel
     for (int t = wave; t < T; t += 16) {
       int si[MAX_TOPK];
@@ -1502,22 +1503,22 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeDev a) {
     __syncthreads();
   }
   // each pair's expert (one round of loads) into LDS, then its token's combine slot from there
-  int pe[(GRP_MAX_PAIRS + 1023) / 1024], idv[(GRP_MAX_PAIRS + 1023) / 1024];
+  int pe[MAXP / 1024], idv[MAXP / 1024];
 #pragma unroll
-  for (int i = 0; i < (GRP_MAX_PAIRS + 1023) / 1024; ++i)  // every id load at once (clamped, unpredicated: under
+  for (int i = 0; i < MAXP / 1024; ++i)  // every id load at once (clamped, unpredicated: under
     idv[i] = a.ids[min(tid + 1024 * i, P - 1)];             // the branches below each would be a round trip)
 #pragma unroll
-  for (int i = 0; i < (GRP_MAX_PAIRS + 1023) / 1024; ++i) {
+  for (int i = 0; i < MAXP / 1024; ++i) {
     const int p = tid + 1024 * i;
     pe[i] = p < P ? (a.topk_in_sort ? (int)s_exp[p] : clamp_expert(idv[i], E)) : 0;
   }
   __syncthreads();  // (every read of s_exp above is done before it is written)
 #pragma unroll
-  for (int i = 0; i < (GRP_MAX_PAIRS + 1023) / 1024; ++i)
+  for (int i = 0; i < MAXP / 1024; ++i)
     if (tid + 1024 * i < P) s_exp[tid + 1024 * i] = (uint8_t)pe[i];
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < (GRP_MAX_PAIRS + 1023) / 1024; ++i) {
+  for (int i = 0; i < MAXP / 1024; ++i) {
     const int p = tid + 1024 * i;
     if (p >= P) break;
     const int t = p / k, j = p - t * k;
@@ -1578,7 +1579,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(MoeDev a) {
         isn += on;
       }
     }
-    const bool gi = a.gu_items != nullptr;  // (t64 layers only: the MXFP4 grouped kernels' items and XCD runs)
+    const bool gi = a.gu_items != nullptr;  // (the 64-token items and XCD runs)
     if (gi) {
       for (int d = 1; d < 64; d <<= 1) {
         int oa[4], od[4];
@@ -3382,6 +3383,266 @@ __global__ __launch_bounds__(256, GU ? 2 : 3) void moe_q4k_mfma_kernel(MoeDev a)
 }
 
 // ---------------------------------------------------------------------------
+// Grouped Q4_K for prompts (many tokens per expert): the same products as
+// moe_q4k_mfma_kernel, in the same order per (pair, row), so the same bits, but
+// each decoded weight multiplies up to 64 tokens instead of 16.
+//
+// Workgroup = (item of up to 64 tokens, 256 rows: gate/up 128 of each), 4
+// waves, one per SIMD with its 512 registers: a wave holds four 16-row tiles
+// (gate/up: two of gate and the same two of up) x the item's token tiles, the
+// sums of the super-block (accumulator registers) and of all of them. Per
+// super-block the wave's codes come from memory a super-block ahead; the tokens'
+// terms (1 KB each, and their sub-block sums) are requested a super-block ahead
+// into registers and parked in the other of two LDS buffers after the products.
+// Nothing but the instruction order hides the decode and the LDS reads: a
+// quarter's terms are read during the quarter before, a row tile's operands are
+// decoded during the tile before's products, the scales and sums likewise.
+//
+// Bound: the matrix cores (18 instructions per 16 rows, 16 tokens and
+// super-block: 250 us of the gate/up launch below), five VALU instructions
+// beside each, and half of a super-block's products ahead of its codes'
+// arrival (the same launch without loads: 598 us). Measured, 1024 tokens of a
+// 128-expert top-8 layer of 4096 x 1536: gate/up 817 us, down 476, against 1876
+// and 1006 with 16-token items.
+constexpr int QG_T = GRP_GU_T;                // tokens per item
+constexpr int QG_TOK = 1024 + 16;             // LDS bytes from token to token: terms, and 16 so that 16 tokens' reads miss
+                                              // each other's banks
+constexpr int QG_SUMS = QG_T * QG_TOK;        // the sub-block sums behind them, 32 bytes a token
+constexpr int QG_BUF = QG_SUMS + QG_T * 32;   // one of two buffers
+constexpr int QG_TILES = 4;                   // 16-row tiles per wave
+constexpr int QG_WAVES = 4;
+constexpr int QG_ROWS = QG_WAVES * QG_TILES * MQ_ROWS;  // rows per workgroup (gate/up: half of them gate, half up)
+
+struct QgW {  // a wave's codes of a super-block, the next one's headers
+  v4u H[QG_TILES], A[QG_TILES], B[QG_TILES], N[QG_TILES];
+};
+
+template <bool GU, int NT>
+__device__ __forceinline__ void qg_run(const MoeDev& a, const int4 item, int unit, uint8_t* xs) {
+  const int NR = GU ? a.n_ff : a.n_embd, K = GU ? a.n_embd : a.n_ff;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
+  const int lr = lane & 15, g = lane >> 4;
+  const int e = clamp_expert(item.x, a.E), pos0 = item.y, n = item.z;
+  // first row of the wave's tiles (tile j: r0 + 16 j; gate/up: tiles 2, 3 are up's rows of tiles 0, 1)
+  const int r0 = (unit * QG_WAVES + wave) * (GU ? 2 : 4) * MQ_ROWS;
+  const int nsb = K / 256;
+  const int64_t rb = (int64_t)nsb * 144, tb = mq_row_bytes(K);
+  const __amdgpu_buffer_rsrc_t rs0 = nsx_rsrc(
+      expert_base(GU ? a.gate_base : a.down_base, GU ? a.gate_stride : a.down_stride, GU ? a.gate_ptrs : a.down_ptrs, e),
+      (uint32_t)(NR * rb));
+  const __amdgpu_buffer_rsrc_t rs1 =
+      GU ? nsx_rsrc(expert_base(a.up_base, a.up_stride, a.up_ptrs, e), (uint32_t)(NR * rb)) : rs0;
+  uint32_t woff[QG_TILES];
+#pragma unroll
+  for (int j = 0; j < QG_TILES; ++j) woff[j] = (uint32_t)(min(r0 + (GU ? j & 1 : j) * MQ_ROWS + lr, NR - 1) * rb);
+  // part p (0: the codes of quarters 0 and 1, 1: those of 2 and 3, 2: the headers) of super-block sb
+  auto load_w = [&](int sb, int part, v4u (&to)[QG_TILES]) {
+    const uint32_t o = part == 2 ? 0u : 16u + 64u * (uint32_t)part + 16u * (uint32_t)g;
+#pragma unroll
+    for (int j = 0; j < QG_TILES; ++j)
+      to[j] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(GU && j >= 2 ? rs1 : rs0, woff[j] + o, sb * 144, 0));
+  };
+  // Lane i knows pair i of the item (pairs past it repeat the last: their columns are not stored) and its term row.
+  const int my_pair = a.sorted[pos0 + min(lane, n - 1)], my_row = GU ? my_pair / a.top_k : my_pair;
+  const uint8_t* tbase = GU ? a.xq_h : (const uint8_t*)a.xq_a;
+  // Terms of a super-block: wave w takes tokens w, w + 4, ... of the NT tiles, a KB each (lanes 0..31 the hi terms,
+  // 32..63 the lo ones), and 32 lanes of each wave the sums of 16 tokens.
+  // In LDS a token's terms lie by lane group (256 bytes each), quarter and operand (low nibbles' hi and lo terms, high
+  // nibbles'): a read instruction's lanes then differ in bank by the token alone.
+  v4u st[2 * NT], ss;
+  const int c8 = lane & 31, pr8 = c8 >> 3, rr = c8 & 3;  // 8 elements 64 pr8 + 32 (c8 / 4 % 2) + 8 rr ..
+  const uint32_t st_off = lane < 32 ? 16u * (uint32_t)lane : 2u * (uint32_t)K + 16u * (uint32_t)(lane - 32);
+  const int st_to = 256 * (2 * (pr8 & 1) + (rr >> 1)) + 64 * (2 * (pr8 >> 1) + (rr & 1)) + 32 * ((c8 >> 2) & 1) + 16 * (lane >> 5);
+  const int s_tok = wave * 16 + ((lane >> 1) & 15);
+  const uint32_t my_off = (uint32_t)my_row * (uint32_t)tb;  // (P rows of terms: below 4 GB)
+  const uint32_t ss_off = (uint32_t)__shfl((int)my_off, s_tok, 64) + 4u * (uint32_t)K + (uint32_t)(lane & 1) * ((uint32_t)K / 16u);
+  const __amdgpu_buffer_rsrc_t rt = nsx_rsrc(tbase, (uint32_t)((int64_t)(GU ? a.T : a.T * a.top_k) * tb));
+  // (half of the tokens at a time, each half requested half a super-block's products before it is parked)
+  auto load_t = [&](int sb, int half) {
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) {
+      const int tok = QG_WAVES * (i + half * 2 * NT) + wave;
+      st[i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(
+          rt, st_off, __builtin_amdgcn_readlane((int)my_off, tok) + sb * 512, 0));
+    }
+    if (half == 0) ss = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rt, ss_off, 16 * sb, 0));
+  };
+  auto park_t = [&](uint8_t* buf, int half) {
+    uint8_t* to = buf + wave * QG_TOK + st_to;
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) *(v4u*)(to + QG_WAVES * (i + half * 2 * NT) * QG_TOK) = st[i];
+    if (half == 0 && lane < 32) *(v4u*)(buf + QG_SUMS + s_tok * 32 + (lane & 1) * 16) = ss;
+  };
+  mq_f4 y[QG_TILES][NT];
+#pragma unroll
+  for (int j = 0; j < QG_TILES; ++j)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) y[j][t] = mq_f4{0.f, 0.f, 0.f, 0.f};
+  // super-block sb's products from `buf`; super-block ns's codes and terms requested, the terms parked in `other`. A half's
+  // codes are requested as soon as the half is decoded (a second set of registers for them, requested a whole
+  // super-block ahead: the gate/up launch 879 us against 817).
+  QgW w;
+  auto compute = [&](int ns, const uint8_t* buf, uint8_t* other) {
+    const mq_h2 k1024 = {(_Float16)1024.f, (_Float16)1024.f}, km1024 = {(_Float16)-1024.f, (_Float16)-1024.f};
+    MqScales S[QG_TILES];
+    mq_f4 acc[QG_TILES][NT];
+#pragma unroll
+    for (int j = 0; j < QG_TILES; ++j)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[j][t] = mq_f4{0.f, 0.f, 0.f, 0.f};
+    const uint8_t* xb = buf + lr * QG_TOK + 256 * g;
+    mq_h8 B[2][NT][4], SH[NT], SL[NT];  // a quarter's terms (and the next one's); the sums
+    auto terms = [&](int q, int t) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) B[q & 1][t][k] = *(const mq_h8*)(xb + 16 * t * QG_TOK + 64 * q + 16 * k);
+    };
+    mq_h8 alo[2], ahi[2];
+    auto decode = [&](int q, int j, int to) {
+      if (q == 0) S[j] = mq_scales(w.H[j], g);
+      const int u = q >> 1;  // (the offsets again each time: their registers are worth more)
+      mq_a_pair(mq_codes(w.A[j], w.B[j], q), S[j].ml[u], S[j].ml[u] * km1024, S[j].mh[u], S[j].mh[u] * km1024, alo[to],
+                ahi[to]);
+    };
+    // tile j's minima and scales (mq_finish, its row factors formed once for all token tiles)
+    auto finish = [&](int j) {
+      const uint32_t m01 = __builtin_bit_cast(uint32_t, mq_biased(S[j].MN03, 0x04010400u) - k1024);
+      const uint32_t m23 = __builtin_bit_cast(uint32_t, mq_biased(S[j].MN03, 0x04030402u) - k1024);
+      const uint32_t m45 = __builtin_bit_cast(uint32_t, mq_biased(S[j].MN47, 0x04010400u) - k1024);
+      const uint32_t m67 = __builtin_bit_cast(uint32_t, mq_biased(S[j].MN47, 0x04030402u) - k1024);
+      const mq_h8 A2 = __builtin_bit_cast(mq_h8, g == 0 ? v4u{m01, m23, m45, m67} : v4u{0u, 0u, 0u, 0u});
+      mq_f4 am[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) am[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2, SH[t], mq_f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) am[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2, SL[t], am[t], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // d, dmin of row 4 g + i: the header lane (4 g + i) loaded
+        const uint32_t dw = (uint32_t)__shfl((int)w.H[j].x, 4 * g + i, 64);
+        const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(dw & 0xFFFFu));
+        const float dm = (float)__builtin_bit_cast(_Float16, (uint16_t)(dw >> 16));
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          y[j][t][i] = fmaf(d, acc[j][t][i], y[j][t][i]);
+          y[j][t][i] = fmaf(-dm, am[t][i], y[j][t][i]);
+        }
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < NT; ++t) terms(0, t);
+    decode(0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int j = 0; j < QG_TILES; ++j) {
+        const int at = q * QG_TILES + j, c = at & 1;
+        if (at + 1 < 4 * QG_TILES) decode((at + 1) / QG_TILES, (at + 1) % QG_TILES, c ^ 1);
+        if (q < 3 && j < NT) terms(q + 1, j);
+        if (q == 2 && j < NT) {
+          SH[j] = *(const mq_h8*)(buf + QG_SUMS + (16 * j + lr) * 32);
+          SL[j] = *(const mq_h8*)(buf + QG_SUMS + (16 * j + lr) * 32 + 16);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k < 2 ? alo[c] : ahi[c], B[q & 1][t][k], acc[j][t], 0, 0, 0);
+        if (q == 3 && j > 0) finish(j - 1);
+#pragma unroll
+        for (int i = 0; i < (q == 3 && j > 0 ? 6 : 4) * NT; ++i) {  // a product, VALU work; a read every few of them
+          if (i % NT == 0) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (q == 0 || (q == 3 && j > 0)) __builtin_amdgcn_sched_group_barrier(0x002, 16 / NT + 1, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x002, 9 / NT + 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (q == 1 && j == QG_TILES - 1) {  // the first half's codes are decoded (the second half's: at q == 3)
+          load_w(ns, 0, w.A);
+          park_t(other, 0);
+          load_t(ns, 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (q == 3 && j == QG_TILES - 2) {
+          load_w(ns, 1, w.B);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    finish(QG_TILES - 1);
+  };
+  load_t(0, 0);
+  load_w(0, 0, w.A);
+  load_w(0, 2, w.H);
+  load_w(0, 1, w.B);
+  park_t(xs, 0);
+  load_t(0, 1);
+  park_t(xs, 1);
+  grp_lds_barrier();
+  // The other buffer is parked in while every wave multiplies from this one; the barrier ends both. The last step
+  // requests super-block nsb - 1 again, and drops it.
+  for (int sb = 0; sb < nsb; ++sb) {
+    const int ns = min(sb + 1, nsb - 1);
+    uint8_t* other = xs + ((sb & 1) ^ 1) * QG_BUF;
+    load_t(ns, 0);
+    load_w(ns, 2, w.N);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(ns, xs + (sb & 1) * QG_BUF, other);
+    __builtin_amdgcn_sched_barrier(0);
+    park_t(other, 1);
+#pragma unroll
+    for (int j = 0; j < QG_TILES; ++j) w.H[j] = w.N[j];
+    grp_lds_barrier();
+  }
+  // (n_ff and n_embd are multiples of 256: every tile is whole, its four rows of a lane 16-byte aligned)
+  if (r0 >= NR) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int tok = 16 * t + lr;
+    const int pr = __shfl(my_pair, tok, 64), row = __shfl(my_row, tok, 64);
+    if (tok >= n) continue;
+    const float scale = *(const float*)(tbase + (int64_t)row * tb + 4 * K + K / 8);  // 2^e of this column's terms
+#pragma unroll
+    for (int j = 0; j < (GU ? 2 : QG_TILES); ++j) {
+      const int r = r0 + j * MQ_ROWS + 4 * g;
+      v4f v;
+      if constexpr (GU) {
+        const float* gb = a.gate_bias ? a.gate_bias + (int64_t)e * a.n_ff + r : nullptr;
+        const float* ub = a.up_bias ? a.up_bias + (int64_t)e * a.n_ff + r : nullptr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float gv = y[j][t][i] * scale, uv = y[(j + 2) % QG_TILES][t][i] * scale;
+          if (gb) gv += gb[i];
+          if (ub) uv += ub[i];
+          v[i] = moe_act(a.act_kind, gv, uv, a.alpha, a.limit);
+        }
+        *(v4f*)(a.act + (int64_t)pr * a.n_ff + r) = v;
+      } else {
+        const float* db = a.down_bias ? a.down_bias + (int64_t)e * a.n_embd + r : nullptr;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = db ? y[j][t][i] * scale + db[i] : y[j][t][i] * scale;
+        *(v4f*)(a.y + (int64_t)pr * a.n_embd + r) = v;
+      }
+    }
+  }
+}
+
+// Workgroup b runs on XCD b % 8: XCD x takes items x, x + 8, ... of the list (heavy first), an item's units next to each
+// other, so that its L2 keeps the item's term rows.
+template <bool GU>
+__global__ __launch_bounds__(64 * QG_WAVES, 1) void moe_q4k_gemm_kernel(MoeDev a) {
+  extern __shared__ __align__(16) uint8_t qg_xs[];  // 2 * QG_BUF
+  const int units = (GU ? 2 * a.n_ff : a.n_embd) / QG_ROWS, live = a.gu_bounds[8] / (int)a.ggu.tiles;
+  const int j = (int)(blockIdx.x >> 3), it = (j / units) * 8 + (int)(blockIdx.x & 7);
+  if (it >= live) return;
+  const int4 item = a.gu_items[it];
+  const int unit = j % units, nt = (item.z + 15) / 16;
+  if (nt <= 1) qg_run<GU, 1>(a, item, unit, qg_xs);
+  else if (nt == 2) qg_run<GU, 2>(a, item, unit, qg_xs);
+  else if (nt == 3) qg_run<GU, 3>(a, item, unit, qg_xs);
+  else qg_run<GU, 4>(a, item, unit, qg_xs);
+}
+
+// ---------------------------------------------------------------------------
 // host side
 
 struct MoePlan {
@@ -3392,6 +3653,7 @@ struct MoePlan {
   bool grouped;
   int max_items, max_gu_items, cdg, sdg;
   bool mq;  // grouped Q4_K on the matrix cores: xqh / xqa hold activation terms (mq_row_bytes per row)
+  bool qg;  // ... with items of up to QG_T tokens (moe_q4k_gemm_kernel)
 };
 
 // NSX_DISPATCH_AUTO groups t64 layers from GRP_AUTO_MIN_T tokens (the 36-layer GPT-OSS stack at T = 2 / 3 / 5 / 7:
@@ -3401,6 +3663,10 @@ struct MoePlan {
 // matrix cores, whose lead grows with the tokens per expert
 constexpr int GRP_AUTO_MIN_T = 3;
 constexpr int MQ_AUTO_MIN_PAIRS = 104;
+// Q4_K on the matrix cores takes the 64-token items from this many pairs per expert on (top-8 of 128, 16-token items /
+// these: 4096 x 1536 at T = 64 442 / 465 us, 96 526 / 481, 128 587 / 485, 1024 2617 / 1300; 2048 x 768 at T = 64
+// 153 / 161, 96 176 / 164, 1024 805 / 432).
+constexpr int QG_MIN_PER_EXPERT = 5;
 
 // The Q4_K kernels take K <= 4096 and 16-byte aligned expert rows.
 static bool q4k_fast(const nsx_moe_layer* L) {
@@ -3435,6 +3701,7 @@ static MoePlan moe_plan(const nsx_moe_layer* L, int64_t T) {
   p.mq = use_mq(L, T);
   if (p.grouped) T = std::min(T, grp_chunk_tokens(L));
   const int64_t P = T * L->top_k;
+  p.qg = p.mq && P >= QG_MIN_PER_EXPERT * L->n_expert;
   const bool t64 = L->layout == NSX_LAYOUT_T64;
   p.ggu = mx_geom(L->n_ff, L->n_embd);
   p.gdn = mx_geom(L->n_embd, L->n_ff);
@@ -3445,7 +3712,7 @@ static MoePlan moe_plan(const nsx_moe_layer* L, int64_t T) {
   p.cdg = std::max(1, std::min(p.gdn.ns, 4));  // grouped down: 4 row groups x cdg chunks
   p.sdg = (int)nsx_cdiv(p.gdn.ns, p.cdg);
   p.max_items = p.grouped ? grp_max_items(L->n_expert, (int)P) : 0;
-  p.max_gu_items = p.grouped && t64 ? grp_max_items(L->n_expert, (int)P, GRP_GU_T) : 0;
+  p.max_gu_items = p.grouped && (t64 || p.qg) ? grp_max_items(L->n_expert, (int)P, GRP_GU_T) : 0;
   auto al = [](int64_t x) { return (x + 255) & ~(int64_t)255; };
   int64_t o = 0;
   p.off_logits = o;
@@ -3660,6 +3927,14 @@ static MoeDev make_dev(const nsx_moe_layer* L, const MoePlan& p, char* ws, const
   return d;
 }
 
+template <bool GU>
+static int launch_qg(const MoePlan& p, const MoeDev& d, int rows, hipStream_t st) {
+  const void* k = (const void*)moe_q4k_gemm_kernel<GU>;
+  NSX_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * QG_BUF));
+  const unsigned grid = (unsigned)(8 * nsx_cdiv(p.max_gu_items, 8) * (rows / QG_ROWS));
+  return nsx_launch(moe_q4k_gemm_kernel<GU>, dim3(grid), dim3(64 * QG_WAVES), (size_t)(2 * QG_BUF), st, d);
+}
+
 // Phases ph0..ph1 of one layer (NSX_PHASE_*); each later phase reads what
 // the earlier ones left in the workspace.
 static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out, int32_t* ids, float* weights,
@@ -3710,7 +3985,9 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
     if (on(NSX_PHASE_GATE_UP)) {
       // a small batch whose top-k the sort would select: the t64 gate/up workgroups sort the pairs themselves
       const bool sin = t64 && d.topk_in_sort && P <= GRP_SMALL_P;
-      if (!sin && (rc = nsx_launch(moe_sort_kernel, dim3(1), dim3(1024), 0, st, d))) return rc;
+      if (!sin && (rc = P <= GRP_SORT_SMALL ? nsx_launch(moe_sort_kernel<GRP_SORT_SMALL>, dim3(1), dim3(1024), 0, st, d)
+                                            : nsx_launch(moe_sort_kernel<GRP_MAX_PAIRS>, dim3(1), dim3(1024), 0, st, d)))
+        return rc;
       if (t64) {
         // persistent: the resident workgroups (a multiple of 8), no more than the units can use
         const void* kern = sin ? (const void*)moe_gu_grouped_kernel<true> : (const void*)moe_gu_grouped_kernel<false>;
@@ -3724,8 +4001,11 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
             (rc = nsx_launch(mq_terms_kernel, dim3((unsigned)T), dim3(256), 0, st, h, (int)L->n_embd,
                              (uint8_t*)(ws + p.off_xqh))))
           return rc;
-        rc = nsx_launch(moe_q4k_mfma_kernel<true>, grid8(nsx_cdiv(L->n_ff, MQ_WG_ROWS)), dim3(256),
-                        (size_t)(MQ_LDS_NT * mq_lds_row(L->n_embd)), st, d);
+        if (p.qg)
+          rc = launch_qg<true>(p, d, 2 * L->n_ff, st);
+        else
+          rc = nsx_launch(moe_q4k_mfma_kernel<true>, grid8(nsx_cdiv(L->n_ff, MQ_WG_ROWS)), dim3(256),
+                          (size_t)(MQ_LDS_NT * mq_lds_row(L->n_embd)), st, d);
       } else {  // Q4_K on the int8 dot: the tokens' activation terms, then the rows
         if ((rc = nsx_launch(a8_terms_kernel, dim3((unsigned)T), dim3(256), 0, st, h, (int)L->n_embd,
                              (uint8_t*)(ws + p.off_xqh))))
@@ -3751,8 +4031,11 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
         if ((rc = nsx_launch(mq_terms_kernel, dim3((unsigned)P), dim3(256), 0, st, (const float*)d.act,
                              (int)L->n_ff, d.xq_a)))
           return rc;
-        rc = nsx_launch(moe_q4k_mfma_kernel<false>, grid8(nsx_cdiv(L->n_embd, 2 * MQ_WG_ROWS)), dim3(256),
-                        (size_t)(MQ_LDS_NT * mq_lds_row(L->n_ff)), st, d);
+        if (p.qg)
+          rc = launch_qg<false>(p, d, L->n_embd, st);
+        else
+          rc = nsx_launch(moe_q4k_mfma_kernel<false>, grid8(nsx_cdiv(L->n_embd, 2 * MQ_WG_ROWS)), dim3(256),
+                          (size_t)(MQ_LDS_NT * mq_lds_row(L->n_ff)), st, d);
       } else {
         if ((rc = nsx_launch(a8_terms_kernel, dim3((unsigned)P), dim3(256), 0, st, (const float*)d.act,
                              (int)L->n_ff, d.xq_a)))

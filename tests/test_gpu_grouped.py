@@ -259,3 +259,42 @@ def test_config4_qwen3_t32_mfma(config4_t32):
     assert torch.equal(im, c["ip"])
     assert rel_max(to_np(om), to_np(c["op"])) < Q4K_TOL
     _check_all_tokens(cfg, t, h, im, wm, om, 1e-5, oracle=c["oracle"])
+
+
+@pytest.mark.parametrize("n_embd,n_ff,T,bias", [(512, 256, 300, False), (512, 768, 41, True), (1024, 512, 1100, False)])
+def test_mfma_q4k_large_batches_equal_small_ones(dev, n_embd, n_ff, T, bias):
+    """Q4_K with at least 5 pairs per expert runs 64-token items (one to four token tiles, experts of
+    several items, an odd number of super-blocks, more pairs than one sort takes); slices of at most 7
+    tokens (56 pairs of 12 experts) run the 16-token items. Each (pair, row) is the same sequence of
+    operations: identical outputs."""
+    from nurostream_amd import synth
+    cfg = synth.MoEConfig("q4k", synth.GGMLType.Q4_K, 12, 8, n_embd, n_ff, "qwen3", "silu_mul", bias, torch.float32)
+    t = synth.make_layer(cfg, seed=29, device=dev)
+    layer = _layer(cfg, t, "gguf", dispatch="mfma")
+    h = synth.activations(T, n_embd, seed=T, device=dev) * torch.linspace(0.01, 30, T, device=dev)[:, None]
+    out, ids, wts = layer(h)
+    for t0 in [*range(0, min(T, 84), 7), T // 2, T - 7]:
+        o, i, w = layer(h[t0:t0 + 7])
+        n = o.shape[0]
+        same = (ids[t0:t0 + n] == i).all(1)  # (the routers of large and small batches sum in different orders)
+        assert int(same.sum()) >= n - 1
+        # the routing weights differ by fp32 rounding with those sums, the expert outputs not at all
+        torch.testing.assert_close(out[t0:t0 + n][same], o[same], rtol=0, atol=2e-6 * float(o.abs().max()))
+    ref, _, _, _ = _oracle_layer(cfg, t, h[:40].cpu().numpy())
+    assert rel_max(to_np(out[:40]), ref) < 1e-5
+
+
+def test_q4k_gemm_kernel_bitwise(dev):
+    """The same with a router that gives every token the same experts and weights in any batch: the outputs of
+    each token compared bit for bit between one call of 63 tokens and nine of 7."""
+    from nurostream_amd import synth
+    cfg = _small("qwen3-small")
+    t = synth.make_layer(cfg, seed=31, device=dev)
+    t["router_w"] = torch.zeros_like(t["router_w"])  # every token: experts 0..7, equal weights, in any batch
+    layer = _layer(cfg, t, "gguf", dispatch="mfma")
+    h = synth.activations(63, cfg.n_embd, seed=2, device=dev)
+    out, ids, _ = layer(h)
+    assert set(ids.unique().tolist()) == set(range(8))
+    for t0 in range(0, 63, 7):
+        o, _, _ = layer(h[t0:t0 + 7])
+        assert torch.equal(out[t0:t0 + 7], o), t0
