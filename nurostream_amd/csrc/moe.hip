@@ -2173,6 +2173,228 @@ __global__ __launch_bounds__(256, 2) void moe_down_persistent_kernel(MoeDev a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Grouped MXFP4 for prompts (many tokens per expert): each (matrix, chunk, 64-row tile) is the MFMA sequence of the
+// kernels above and the chunks' sums are added in the same order, so the bits do not depend on the dispatch.
+//
+// The kernels above split K over a workgroup's waves, so that each wave reads a token's terms of its chunk from L2 for
+// 64 rows (128 with gate and up): at many tokens per expert those reads (4.5 bytes per element and token, 36 bytes a
+// clock and CU) set the time, the matrix cores busy for 29 % of it. Here a workgroup is (item of up to 64 tokens, 4 row
+// tiles), a wave a tile (gate/up: waves 0, 1 gate, 2, 3 the same tiles of up): it walks K chunk by chunk, a chunk's
+// terms go into LDS once for the four waves, 16 tokens at a time and without passing registers (gate/up: two buffers,
+// the next 16 tokens requested before these products; the down chunk of six steps has LDS for one, its waits covered by
+// the CU's other workgroup), a wave's weights of the chunk stay in registers over all tokens, and the sums of the chunks
+// stay there to the end. The sum over the four terms is the pairs of mx_sum_terms, each group of four tokens' kept by
+// one lane of a quad: 2.5 instructions a product instead of 4.
+//
+// Bound: the matrix cores (4 terms a token: 32 cycles per 16 rows, 4 tokens and K-step; busy for 40 % of the time) and
+// the VALU beside them (sums, then SwiGLU and the split into terms; 45 %), two waves a SIMD for both. 2880 x 2880, 128
+// experts, T = 2048: gate/up 892 -> 792 us, down 410 -> 370. Tried and no faster: the weights of the next chunk
+// requested into the L2 ahead (gate/up 801, down 398), a group's sums scheduled beside the next group's products (785,
+// 32 experts slower), eight waves a workgroup with the terms through registers (1032, 404).
+constexpr int XG_WAVES = 4;
+constexpr int XG_T = GRP_GU_T;     // tokens per item
+constexpr int XG_TOK = 16;         // tokens of a stage
+constexpr int XG_STEP = 9 * 1024;  // LDS bytes of a step: [half][lane group][token][term][16 B], then the scales,
+                                   // [token / 4][lane group][token % 4][term][4 B]
+template <bool GU>
+struct XgShape {
+  static constexpr int S = GU ? GU_S : DC_S;  // K-steps of a chunk
+  static constexpr int NBUF = GU ? 2 : 1;
+  static constexpr int BUF = S * XG_STEP;
+  static constexpr int LOADS = (9 * S + XG_WAVES - 1) / XG_WAVES;  // a wave's loads of a stage, 1 KB each
+};
+// (gate/up: at the end gate's and up's sums of all tokens meet in LDS)
+constexpr int XG_LDS = XG_WAVES * XG_T * 64 * 4;
+static_assert(2 * GU_S * XG_STEP <= XG_LDS && DC_S * XG_STEP <= XG_LDS, "the stages fit the epilogue's LDS");
+
+template <bool GU>
+__global__ __launch_bounds__(64 * XG_WAVES, 2) void moe_mx_gemm_kernel(MoeDev a) {
+  using X = XgShape<GU>;
+  constexpr int S = X::S;
+  extern __shared__ __align__(16) uint8_t xg_xs[];
+  const MxGeom& G = GU ? a.ggu : a.gdn;
+  constexpr int TPU = GU ? XG_WAVES / 2 : XG_WAVES;  // row tiles of a unit
+  const int tiles = (int)G.tiles, units = (tiles + TPU - 1) / TPU, live = a.gu_bounds[8] / (int)a.ggu.tiles;
+  // workgroup b runs on XCD b % 8: XCD x takes items x, x + 8, ... (heavy first), an item's units next to each other,
+  // so that its L2 keeps the item's terms
+  const int jb = (int)(blockIdx.x >> 3), it = (jb / units) * 8 + (int)(blockIdx.x & 7);
+  if (it >= live) return;
+  const int4 item = a.gu_items[it];
+  const int e = clamp_expert(item.x, a.E), n = item.z;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
+  const int tile = (jb % units) * TPU + (GU ? wave % TPU : wave), tc = min(tile, tiles - 1);
+  const bool up = GU && wave >= TPU;
+  const uint8_t* mat = !GU  ? tile_base(a.down_base, a.down_stride, a.down_ptrs, a.down_tiles, G, e, tc)
+                       : up ? tile_base(a.up_base, a.up_stride, a.up_ptrs, a.up_tiles, G, e, tc)
+                            : tile_base(a.gate_base, a.gate_stride, a.gate_ptrs, a.gate_tiles, G, e, tc);
+  const int sg = GU ? a.sg : a.sdg, nch = GU ? a.cg : a.cdg;
+  // lane i: pair i of the item (pairs past it repeat the last; their columns are not stored)
+  const int my_pair = a.sorted[item.y + min(lane, n - 1)];
+  const int64_t xs = (int64_t)G.ns * XQ_STEP;
+  const uint32_t my_off = (uint32_t)((int64_t)(GU ? my_pair / a.top_k : my_pair) * xs);
+  const __amdgpu_buffer_rsrc_t rt =
+      nsx_rsrc(GU ? a.xq_h : (const uint8_t*)a.xq_a, (uint32_t)((int64_t)(GU ? a.T : a.T * a.top_k) * xs));
+  // Stage (chunk c, part p): tokens 16 p .. + 15, the chunk's steps, 1 KB a wave load straight into LDS. Lane l takes
+  // token l / 4, term l % 4 of a code plane, or token 4 (l / 16) + l % 4, lane group l / 4 % 4 of the scales.
+  typedef __attribute__((address_space(3))) void lds_void;
+  auto fill = [&](int c, int p, int buf) {
+    const uint32_t vc = (uint32_t)__shfl((int)my_off, 16 * p + (lane >> 2), 64) + 32u * (uint32_t)(lane & 3);
+    const uint32_t vs =
+        (uint32_t)__shfl((int)my_off, 16 * p + 4 * (lane >> 4) + (lane & 3), 64) + 16u * (uint32_t)((lane >> 2) & 3);
+#pragma unroll
+    for (int i = 0; i < X::LOADS; ++i) {
+      const int q = min(wave + XG_WAVES * i, 9 * S - 1);  // (a wave past the last load repeats it)
+      const int step = q / 9, k = q - 9 * step;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rt, (lds_void*)(xg_xs + buf * X::BUF + q * 1024), 16, k < 8 ? vc : vs,
+          min(c * sg + step, G.ns - 1) * XQ_STEP + (k < 8 ? (k & 3) * 128 + (k >> 2) * 16 : XQ_CODES), 0, 0);
+    }
+  };
+  v4f y[XG_T / 16][4];
+#pragma unroll
+  for (int p = 0; p < XG_T / 16; ++p)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) y[p][g] = v4f{0.f, 0.f, 0.f, 0.f};
+  MxRegs<S> R;
+  // A stage's products: four tokens at a time (16 columns = 4 tokens x 4 terms). Each group's sum over the terms (the
+  // pairs of mx_sum_terms) is kept by the lanes 4 i + (group): token 16 p + 4 (lane % 4) + lane % 16 / 4, rows
+  // 16 g + 4 (lane / 16) ..
+  const uint32_t lb = (uint32_t)((lane >> 4) * 1024 + (lane & 15) * 16);
+  auto group = [&](int s0, int s1, const uint8_t* buf, int cg, v4f (&D)[4]) {
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+      const uint8_t* x = buf + u * XG_STEP + cg * 256;
+      R.B0[u] = *(const v4u*)(x + lb);
+      R.B1[u] = *(const v4u*)(x + 4096 + lb);
+      R.SB[u] = *(const uint32_t*)(x + 8192 + lane * 4);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) D[g] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (GU && s1 - s0 == S) mx_compute<S>(R, G, 0, S, D);  // (no branch between the steps; six would spill)
+    else mx_compute<S>(R, G, s0, s1, D);
+  };
+  const bool odd = lane & 1, hi = lane & 2;
+  auto pair = [&](int s0, int s1, const uint8_t* buf, int cg, v4f (&r)[4]) {  // the sums over term pairs of two groups of tokens
+    v4f D[4];
+    group(s0, s1, buf, cg, D);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[g][i] = D[g][i] + nsx_dpp_fold<0xB1>(D[g][i]);
+    group(s0, s1, buf, cg + 1, D);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = D[g][i] + nsx_dpp_fold<0xB1>(D[g][i]);
+        r[g][i] = odd ? v : r[g][i];
+      }
+  };
+  auto stage = [&](int c, auto part, const uint8_t* buf) {
+    constexpr int P = decltype(part)::value;
+    const int s0 = c * sg, s1 = min(G.ns, s0 + sg);
+    v4f r[4];
+    pair(s0, s1, buf, 0, r);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = r[g][i] + nsx_dpp_fold<0x4E>(r[g][i]);
+        y[P][g][i] += hi ? 0.f : v;
+      }
+    if (16 * P + 8 >= n) return;
+    pair(s0, s1, buf, 2, r);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = r[g][i] + nsx_dpp_fold<0x4E>(r[g][i]);
+        y[P][g][i] += hi ? v : 0.f;
+      }
+  };
+  // chunk c's weights
+  auto chunk_a = [&](int c) {
+    const int s0 = c * sg;
+    mx_load_a_flat<S>(R, mat, G, s0, min(G.ns, s0 + sg));
+  };
+  auto arrived = []() {  // this wave's LDS loads are in, then every wave's
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    grp_lds_barrier();
+  };
+  fill(0, 0, 0);
+  int flip = 0;
+  for (int c = 0; c < nch; ++c) {
+    chunk_a(c);
+    // part p of the chunk; two buffers: the stage after it is requested before its products
+    auto run = [&](auto part) {
+      constexpr int p = decltype(part)::value;
+      if (16 * p >= n) return;
+      const bool last = p == XG_T / 16 - 1 || 16 * (p + 1) >= n;
+      const int cn = last ? c + 1 : c, pn = last ? 0 : p + 1;
+      arrived();
+      if (X::NBUF == 2 && cn < nch) fill(cn, pn, flip ^ 1);
+      stage(c, part, xg_xs + flip * X::BUF);
+      if (X::NBUF == 2) {
+        flip ^= 1;
+      } else {
+        grp_lds_barrier();
+        if (cn < nch) fill(cn, pn, 0);
+      }
+    };
+    run(std::integral_constant<int, 0>{});
+    run(std::integral_constant<int, 1>{});
+    run(std::integral_constant<int, 2>{});
+    run(std::integral_constant<int, 3>{});
+    if (!GU && c == 0 && a.down_bias) {  // the bias joins chunk 0's sum first
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int r = tc * 64 + 16 * g + 4 * (lane >> 4);
+        const v4f b = r < a.n_embd ? *(const v4f*)(a.down_bias + (int64_t)e * a.n_embd + r) : v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < XG_T / 16; ++p) y[p][g] += b;
+      }
+    }
+  }
+  const int tok0 = 4 * (lane & 3) + ((lane & 15) >> 2);  // this lane's token of each 16
+  if constexpr (!GU) {
+    if (tile >= tiles) return;
+#pragma unroll
+    for (int p = 0; p < XG_T / 16; ++p) {
+      const int tok = 16 * p + tok0, pr = __shfl(my_pair, tok, 64);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int r = tile * 64 + 16 * g + 4 * (lane >> 4);
+        if (tok < n && r < a.n_embd) *(v4f*)(a.y + (int64_t)pr * a.n_embd + r) = y[p][g];
+      }
+    }
+  } else {
+    // gate's and up's sums into LDS, [wave][token][row] (once every wave has left the stages' buffers; the rows' 16-byte
+    // pieces in an order of the token's, so that neither side meets a bank twice); then a wave per (token, tile):
+    // lane = row, two whole 32-element blocks of the down matrix's K
+    float* sums = (float*)xg_xs;
+    const int tt = (jb % units) * TPU + wave % TPU, row = tt * 64 + lane, rowc = min(row, a.n_ff - 1);
+    const float gb = a.gate_bias ? a.gate_bias[(int64_t)e * a.n_ff + rowc] : 0.f;
+    const float ub = a.up_bias ? a.up_bias[(int64_t)e * a.n_ff + rowc] : 0.f;
+    grp_lds_barrier();
+#pragma unroll
+    for (int p = 0; p < XG_T / 16; ++p)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(v4f*)(sums + (wave * XG_T + 16 * p + tok0) * 64 + 4 * ((4 * g + (lane >> 4)) ^ tok0)) = y[p][g];
+    grp_lds_barrier();
+    if (tt >= tiles) return;
+    for (int tok = wave / TPU; tok < n; tok += XG_WAVES / TPU) {
+      const float* gsum = sums + ((wave % TPU) * XG_T + tok) * 64 + (lane ^ (4 * (tok & 15)));
+      const float gs = gsum[0], us = gsum[TPU * XG_T * 64];
+      const float av = row < a.n_ff ? moe_act(a.act_kind, gs + gb, us + ub, a.alpha, a.limit) : 0.f;
+      uint8_t* dst = a.xq_a + (int64_t)__builtin_amdgcn_readlane(my_pair, tok) * a.gdn.ns * XQ_STEP;
+      xq_block(av, 2 * tt + (lane >> 5), dst);
+      xq_zero_tail(tt, a.ggu, a.gdn, dst);
+    }
+  }
+}
+
 // out[t, row] = sum over t's pairs in ascending expert id of w * y (grid: rows/256 x T)
 template <int KMAX>  // top_k <= KMAX: the token's pair indices in one round of loads, then their weights and rows
 __global__ __launch_bounds__(256) void moe_combine_kernel(MoeDev a) {
@@ -3654,6 +3876,7 @@ struct MoePlan {
   int max_items, max_gu_items, cdg, sdg;
   bool mq;  // grouped Q4_K on the matrix cores: xqh / xqa hold activation terms (mq_row_bytes per row)
   bool qg;  // ... with items of up to QG_T tokens (moe_q4k_gemm_kernel)
+  bool xg;  // grouped MXFP4 with items' terms in LDS (moe_mx_gemm_kernel)
 };
 
 // NSX_DISPATCH_AUTO groups t64 layers from GRP_AUTO_MIN_T tokens (the 36-layer GPT-OSS stack at T = 2 / 3 / 5 / 7:
@@ -3667,6 +3890,11 @@ constexpr int MQ_AUTO_MIN_PAIRS = 104;
 // these: 4096 x 1536 at T = 64 442 / 465 us, 96 526 / 481, 128 587 / 485, 1024 2617 / 1300; 2048 x 768 at T = 64
 // 153 / 161, 96 176 / 164, 1024 805 / 432).
 constexpr int QG_MIN_PER_EXPERT = 5;
+// MXFP4 takes moe_mx_gemm_kernel from this many pairs per expert on: below, an item's tokens no longer cover the reads of
+// its weights, chunk by chunk (whole layer, us, the kernels above / these, 2880 x 2880, top-4: 128 experts, T = 512 (16
+// pairs per expert) 504 / 514, 1024 753 / 724, 2048 1246 / 1141; 32 experts, T = 128 158 / 185, 256 233 / 243, 512
+// 378 / 357, 1024 612 / 579, 2048 1151 / 1014).
+constexpr int XG_MIN_PER_EXPERT = 48;
 
 // The Q4_K kernels take K <= 4096 and 16-byte aligned expert rows.
 static bool q4k_fast(const nsx_moe_layer* L) {
@@ -3702,6 +3930,7 @@ static MoePlan moe_plan(const nsx_moe_layer* L, int64_t T) {
   if (p.grouped) T = std::min(T, grp_chunk_tokens(L));
   const int64_t P = T * L->top_k;
   p.qg = p.mq && P >= QG_MIN_PER_EXPERT * L->n_expert;
+  p.xg = p.grouped && L->layout == NSX_LAYOUT_T64 && P >= XG_MIN_PER_EXPERT * L->n_expert;
   const bool t64 = L->layout == NSX_LAYOUT_T64;
   p.ggu = mx_geom(L->n_ff, L->n_embd);
   p.gdn = mx_geom(L->n_embd, L->n_ff);
@@ -3928,6 +4157,14 @@ static MoeDev make_dev(const nsx_moe_layer* L, const MoePlan& p, char* ws, const
 }
 
 template <bool GU>
+static int launch_xg(const MoePlan& p, const MoeDev& d, hipStream_t st) {
+  NSX_HIP(hipFuncSetAttribute((const void*)moe_mx_gemm_kernel<GU>, hipFuncAttributeMaxDynamicSharedMemorySize, XG_LDS));
+  const int64_t units = nsx_cdiv(GU ? p.ggu.tiles : p.gdn.tiles, GU ? XG_WAVES / 2 : XG_WAVES);
+  return nsx_launch(moe_mx_gemm_kernel<GU>, dim3((unsigned)(8 * nsx_cdiv(p.max_gu_items, 8) * units)), dim3(64 * XG_WAVES),
+                    (size_t)XG_LDS, st, d);
+}
+
+template <bool GU>
 static int launch_qg(const MoePlan& p, const MoeDev& d, int rows, hipStream_t st) {
   const void* k = (const void*)moe_q4k_gemm_kernel<GU>;
   NSX_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * QG_BUF));
@@ -3984,11 +4221,13 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
     auto grid8 = [&](int64_t groups) { return dim3((unsigned)(8 * nsx_cdiv(items * groups, 8))); };
     if (on(NSX_PHASE_GATE_UP)) {
       // a small batch whose top-k the sort would select: the t64 gate/up workgroups sort the pairs themselves
-      const bool sin = t64 && d.topk_in_sort && P <= GRP_SMALL_P;
+      const bool sin = t64 && !p.xg && d.topk_in_sort && P <= GRP_SMALL_P;
       if (!sin && (rc = P <= GRP_SORT_SMALL ? nsx_launch(moe_sort_kernel<GRP_SORT_SMALL>, dim3(1), dim3(1024), 0, st, d)
                                             : nsx_launch(moe_sort_kernel<GRP_MAX_PAIRS>, dim3(1), dim3(1024), 0, st, d)))
         return rc;
-      if (t64) {
+      if (p.xg) {
+        rc = launch_xg<true>(p, d, st);
+      } else if (t64) {
         // persistent: the resident workgroups (a multiple of 8), no more than the units can use
         const void* kern = sin ? (const void*)moe_gu_grouped_kernel<true> : (const void*)moe_gu_grouped_kernel<false>;
         const int64_t r = std::max<int64_t>(8, nsx_resident_workgroups(kern, 0, 64 * p.cg) / 8 * 8);
@@ -4019,7 +4258,9 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
       if (rc) return rc;
     }
     if (on(NSX_PHASE_DOWN)) {
-      if (t64) {
+      if (p.xg) {
+        rc = launch_xg<false>(p, d, st);
+      } else if (t64) {
         // persistent (the resident workgroups, a multiple of 8) when its units can number GRP_DN_PERSIST times
         // the resident workgroups, else one workgroup per (GRP_TPI-token item, tile)
         const int64_t r = std::max<int64_t>(

@@ -387,8 +387,8 @@ __device__ __forceinline__ void mx_sum_terms(v4f (&D)[G]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float v = D[g][i];
-      v += nsx_dpp_f<0xB1>(v);  // quad_perm [1,0,3,2]: lane ^ 1
-      v += nsx_dpp_f<0x4E>(v);  // quad_perm [2,3,0,1]: lane ^ 2
+      v += nsx_dpp_fold<0xB1>(v);  // quad_perm [1,0,3,2]: lane ^ 1
+      v += nsx_dpp_fold<0x4E>(v);  // quad_perm [2,3,0,1]: lane ^ 2
       D[g][i] = v;
     }
   }

@@ -298,3 +298,24 @@ def test_q4k_gemm_kernel_bitwise(dev):
     for t0 in range(0, 63, 7):
         o, _, _ = layer(h[t0:t0 + 7])
         assert torch.equal(out[t0:t0 + 7], o), t0
+
+
+@pytest.mark.parametrize("n_embd,n_ff,T,bias,slabs", [(96, 64, 96, False, False),     # one K-step, one tile
+                                                     (320, 224, 131, True, True),    # partial steps, tiles and groups
+                                                     (704, 2880, 200, True, False)])  # six steps a down chunk, then five
+def test_mx_gemm_kernel_bitwise(dev, n_embd, n_ff, T, bias, slabs):
+    """Many tokens per expert (one expert with more than a work item, one with few): the same bits as the per-pair
+    kernels, whose sums over K it repeats (top-4: those split the down product in 16 / top_k chunks, the grouped ones
+    in 4); experts in one tensor and at addresses of their own."""
+    from nurostream_amd import synth
+    cfg = synth.MoEConfig("mx", synth.GGMLType.MXFP4, 8, 4, n_embd, n_ff, "gptoss",
+                          "clamped_swiglu" if bias else "silu_mul", bias, torch.bfloat16)
+    t = synth.make_layer(cfg, seed=17, device=dev)
+    t["router_b"] = torch.tensor([0.0, 0.3, -0.3, 0.0] * 2, device=dev)
+    lp, lg = (_layer(cfg, t, "t64", slabs=slabs, dispatch=d) for d in ("pairs", "grouped"))
+    h = synth.activations(T, cfg.n_embd, seed=T, device=dev)
+    op, ip, _ = lp(h)
+    og, ig, _ = lg(h)
+    n = torch.bincount(ig.flatten().long(), minlength=8)
+    assert n.sum() >= 48 * 8 and n.max() > 64  # (the rule's 48 pairs per expert; a second work item)
+    assert torch.equal(ip, ig) and torch.equal(op, og)
