@@ -53,8 +53,8 @@ enum { NSX_ROUTE_GPTOSS = 0, NSX_ROUTE_QWEN3 = 1 };
 enum { NSX_ACT_CLAMPED_SWIGLU = 0, NSX_ACT_SILU_MUL = 1 };
 /* How nsx_moe_forward runs the routed experts: per (token, expert) pair, or
  * grouped (pairs sorted by expert; each active expert's weights read once per
- * work item of up to 16 of its tokens; t64 MXFP4 layers, and stacked 16-byte
- * aligned Q4_K rows with K <= 4096). MFMA: grouped stacked Q4_K on the
+ * work item of 16, with many tokens per expert 64, of its tokens; t64 MXFP4
+ * layers, and stacked 16-byte aligned Q4_K rows with K <= 4096). MFMA: grouped stacked Q4_K on the
  * matrix cores (f16 products of the exact sc * q codes and a two-term split
  * of the activations; outputs within 1e-5 of the per-pair kernels' rather
  * than identical to them). AUTO groups t64 layers from T >= 3 and takes MFMA
@@ -196,6 +196,10 @@ typedef struct nsx_moe_layer {
  * workspace once before its first use (padding inside it must read as zero);
  * calls that share one workspace must not overlap. */
 int64_t nsx_moe_workspace_bytes(const nsx_moe_layer *L, int64_t T);
+/* The same for grouped passes of up to 8192 (token, expert) pairs, which
+ * nsx_moe_forward and nsx_moe_forward_addnorm run where the workspace holds
+ * one (otherwise passes of 4096; each reads every active expert once). */
+int64_t nsx_moe_workspace_bytes_wide(const nsx_moe_layer *L, int64_t T);
 
 /* out: (T, n_embd) fp32 = sum over the token's experts, in ascending expert
  * id, of weight * expert_ffn(h). ids/weights: (T, top_k) outputs. */

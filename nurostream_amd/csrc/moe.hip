@@ -1415,8 +1415,10 @@ constexpr int GRP_GU_T = 64;         // tokens per MXFP4 gate/up work item (GRP_
 // the resident workgroups (the 36-layer GPT-OSS stack at T = 8, at most 1485 units on 512 workgroups: 23.7 us per
 // layer one workgroup per unit, 25.8 persistent; config 3, T = 128: 89.7 -> 84.5 us persistent)
 constexpr int GRP_DN_PERSIST = 8;
-constexpr int GRP_MAX_PAIRS = 8192;  // pairs per sort (nsx_moe_forward splits larger T)
-constexpr int GRP_SORT_SMALL = 4096;  // up to this many the sort kernel with half the LDS and loads
+constexpr int GRP_MAX_PAIRS = 4096;  // pairs per sort (nsx_moe_forward splits larger T)
+// ... with a workspace for it (nsx_moe_workspace_bytes_wide): a pass reads every active expert again, so as many as the
+// LDS of a sort kernel takes (MXFP4 2880 x 2880, 128 experts, 8192 pairs: two passes 1475 us, one 1260)
+constexpr int GRP_WIDE_PAIRS = 8192;
 
 __host__ __device__ __forceinline__ int grp_max_items(int E, int P, int tpi = GRP_TPI) {
   return (E < P ? E : P) + (P + tpi - 1) / tpi;
@@ -3920,14 +3922,16 @@ static bool use_grouped(const nsx_moe_layer* L, int64_t T) {
   return L->dispatch == NSX_DISPATCH_AUTO && L->layout == NSX_LAYOUT_T64 && T >= GRP_AUTO_MIN_T;
 }
 
-// tokens per grouped pass (the sort handles GRP_MAX_PAIRS pairs)
-static int64_t grp_chunk_tokens(const nsx_moe_layer* L) { return GRP_MAX_PAIRS / std::max(1, (int)L->top_k); }
+// tokens per grouped pass (a sort handles GRP_MAX_PAIRS pairs, the wide one GRP_WIDE_PAIRS)
+static int64_t grp_chunk_tokens(const nsx_moe_layer* L, bool wide = false) {
+  return (wide ? GRP_WIDE_PAIRS : GRP_MAX_PAIRS) / std::max(1, (int)L->top_k);
+}
 
-static MoePlan moe_plan(const nsx_moe_layer* L, int64_t T) {
+static MoePlan moe_plan(const nsx_moe_layer* L, int64_t T, bool wide = false) {
   MoePlan p{};
   p.grouped = use_grouped(L, T);
   p.mq = use_mq(L, T);
-  if (p.grouped) T = std::min(T, grp_chunk_tokens(L));
+  if (p.grouped) T = std::min(T, grp_chunk_tokens(L, wide));
   const int64_t P = T * L->top_k;
   p.qg = p.mq && P >= QG_MIN_PER_EXPERT * L->n_expert;
   p.xg = p.grouped && L->layout == NSX_LAYOUT_T64 && P >= XG_MIN_PER_EXPERT * L->n_expert;
@@ -3980,6 +3984,17 @@ static int check_layer(const nsx_moe_layer* L, int64_t T);
 extern "C" int64_t nsx_moe_workspace_bytes(const nsx_moe_layer* L, int64_t T) {
   if (check_layer(L, T) != NSX_OK) return -1;
   return moe_plan(L, T).total;
+}
+
+extern "C" int64_t nsx_moe_workspace_bytes_wide(const nsx_moe_layer* L, int64_t T) {
+  if (check_layer(L, T) != NSX_OK) return -1;
+  return moe_plan(L, T, true).total;
+}
+
+// tokens per pass of a grouped call of T tokens: wide ones where the workspace holds such a pass
+static int64_t grp_pass_tokens(const nsx_moe_layer* L, int64_t T, int64_t workspace_bytes) {
+  const bool wide = T > grp_chunk_tokens(L) && workspace_bytes >= moe_plan(L, T, true).total;
+  return grp_chunk_tokens(L, wide);
 }
 
 static int check_layer(const nsx_moe_layer* L, int64_t T) {
@@ -4180,7 +4195,7 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
   int rc = check_layer(L, T);
   if (rc) return rc;
   NSX_REQUIRE(h && out && ids && weights && workspace, NSX_EINVAL, "null buffer");
-  const MoePlan p = moe_plan(L, T);
+  const MoePlan p = moe_plan(L, T, true);  // (the caller split T into passes)
   NSX_REQUIRE(workspace_bytes >= p.total, NSX_EINVAL, "workspace of %lld bytes, need %lld",
               (long long)workspace_bytes, (long long)p.total);
   NSX_REQUIRE(T * L->top_k < (1ll << 24), NSX_EINVAL, "too many (token, expert) pairs");
@@ -4222,8 +4237,8 @@ static int moe_run(const nsx_moe_layer* L, const float* h, int64_t T, float* out
     if (on(NSX_PHASE_GATE_UP)) {
       // a small batch whose top-k the sort would select: the t64 gate/up workgroups sort the pairs themselves
       const bool sin = t64 && !p.xg && d.topk_in_sort && P <= GRP_SMALL_P;
-      if (!sin && (rc = P <= GRP_SORT_SMALL ? nsx_launch(moe_sort_kernel<GRP_SORT_SMALL>, dim3(1), dim3(1024), 0, st, d)
-                                            : nsx_launch(moe_sort_kernel<GRP_MAX_PAIRS>, dim3(1), dim3(1024), 0, st, d)))
+      if (!sin && (rc = P <= GRP_MAX_PAIRS ? nsx_launch(moe_sort_kernel<GRP_MAX_PAIRS>, dim3(1), dim3(1024), 0, st, d)
+                                           : nsx_launch(moe_sort_kernel<GRP_WIDE_PAIRS>, dim3(1), dim3(1024), 0, st, d)))
         return rc;
       if (p.xg) {
         rc = launch_xg<true>(p, d, st);
@@ -4328,8 +4343,8 @@ extern "C" int nsx_moe_forward(const nsx_moe_layer* L, const float* h, int64_t T
                                float* weights, void* workspace, int64_t workspace_bytes, void* stream) {
   int rc = check_layer(L, T);
   if (rc) return rc;
-  const int64_t tc = use_grouped(L, T) ? grp_chunk_tokens(L) : T;
-  for (int64_t t0 = 0; t0 < T; t0 += tc) {  // grouped passes of at most GRP_MAX_PAIRS pairs, in token order
+  const int64_t tc = use_grouped(L, T) ? grp_pass_tokens(L, T, workspace_bytes) : T;
+  for (int64_t t0 = 0; t0 < T; t0 += tc) {  // grouped passes in token order
     const int64_t n = std::min(tc, T - t0);
     const int64_t k = L->top_k;
     if (h == nullptr || out == nullptr || ids == nullptr || weights == nullptr)
@@ -4380,7 +4395,7 @@ extern "C" int nsx_moe_forward_addnorm(const nsx_moe_layer* L, const float* h, i
     if ((rc = nsx_moe_forward(L, h, T, h_out, ids, weights, workspace, workspace_bytes, stream))) return rc;
     return nsx_add_rmsnorm(x, h_out, T, L->n_embd, eps, norm_w, x_out, h_out, stream);
   }
-  const int64_t tc = grp_chunk_tokens(L), k = L->top_k, ne = L->n_embd;
+  const int64_t tc = grp_pass_tokens(L, T, workspace_bytes), k = L->top_k, ne = L->n_embd;
   for (int64_t t0 = 0; t0 < T; t0 += tc) {  // grouped passes in token order, as nsx_moe_forward
     const int64_t nt = std::min(tc, T - t0);
     // moe_run plans each pass for its own token count: a short last pass (AUTO: t64 below GRP_AUTO_MIN_T tokens,
@@ -4521,7 +4536,9 @@ extern "C" int nsx_moe_phase(const nsx_moe_layer* L, int phase, const float* h, 
 // race on it.
 
 constexpr int MAX_DEVICES = 64;
-static __device__ __align__(256) uint8_t scratch[NSX_STATIC_WORKSPACE_BYTES];
+// (the 64-token items of a Q4_K layer, under 8 KB, lie past the bytes that decide which T are taken)
+constexpr int64_t STATIC_ITEMS = 16 << 10;
+static __device__ __align__(256) uint8_t scratch[NSX_STATIC_WORKSPACE_BYTES + STATIC_ITEMS];
 static std::mutex scratch_mu;
 static void* scratch_addr[MAX_DEVICES];
 
@@ -4552,8 +4569,9 @@ extern "C" int nsx_moe_forward_static(const nsx_moe_layer* L, const float* h, in
   NSX_REQUIRE(h && out && ids && weights, NSX_EINVAL, "null buffer");
   // nsx_moe_forward runs grouped passes of at most grp_chunk_tokens tokens, each planned for its own size
   const int64_t tc = use_grouped(L, T) ? std::min(T, grp_chunk_tokens(L)) : T;
-  const int64_t need = moe_plan(L, tc).total;
-  NSX_REQUIRE(need <= NSX_STATIC_WORKSPACE_BYTES, NSX_EINVAL,
+  const MoePlan p = moe_plan(L, tc);
+  const int64_t need = p.total, items = p.qg ? std::min(STATIC_ITEMS, (int64_t)p.max_gu_items * 16 + 512) : 0;
+  NSX_REQUIRE(need <= NSX_STATIC_WORKSPACE_BYTES + items, NSX_EINVAL,
               "T=%lld needs a %lld-byte workspace; the static workspace holds %lld bytes (use nsx_moe_forward "
               "with a caller workspace, or fewer tokens per call)",
               (long long)T, (long long)need, (long long)NSX_STATIC_WORKSPACE_BYTES);

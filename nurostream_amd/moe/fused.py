@@ -41,7 +41,7 @@ class MoELayer:
         (expert e at offset e * bytes_per_expert) or a list of n_expert device
         tensors (one slab each). dispatch: "pairs" runs each (token, expert)
         pair on its own, "grouped" sorts the pairs by expert and reads each
-        active expert once per work item of up to 16 tokens (t64 layout),
+        active expert once per work item of up to 16 or 64 tokens (t64 layout),
         "auto" groups from 3 tokens on (t64). These give identical outputs.
         "mfma" groups stacked Q4_K experts and runs them on the matrix cores
         (within 1e-5 of the others, not identical); "auto" takes it for such
@@ -120,7 +120,7 @@ class MoELayer:
     def workspace(self, T: int) -> torch.Tensor:
         ws = self._ws.get(T)
         if ws is None:
-            n = N.load().nsx_moe_workspace_bytes(C.byref(self._c), T)
+            n = N.load().nsx_moe_workspace_bytes_wide(C.byref(self._c), T)
             if n < 0:
                 raise ValueError(f"bad layer for T={T}")
             # zeroed once: padding inside the workspace must read as zero

@@ -319,3 +319,20 @@ def test_mx_gemm_kernel_bitwise(dev, n_embd, n_ff, T, bias, slabs):
     n = torch.bincount(ig.flatten().long(), minlength=8)
     assert n.sum() >= 48 * 8 and n.max() > 64  # (the rule's 48 pairs per expert; a second work item)
     assert torch.equal(ip, ig) and torch.equal(op, og)
+
+
+@pytest.mark.parametrize("name,layout,T", [("gptoss-small", "t64", 2100), ("qwen3-small", "gguf", 1030)])
+def test_wide_passes_equal_narrow_ones(dev, name, layout, T):
+    """More than 8192 pairs in passes of 8192 (the workspace for it), of 4096 (the plain workspace), and the last pass."""
+    import ctypes as C
+    from nurostream_amd import _native as N, synth
+    cfg = _small(name)
+    layer = _layer(cfg, synth.make_layer(cfg, seed=43, device=dev), layout)
+    h = synth.activations(T, cfg.n_embd, seed=T, device=dev)
+    out, ids, w = layer(h)
+    narrow = layer.new_workspace(T)
+    assert T * cfg.top_k > 8192 and layer.workspace(T).numel() > narrow.numel()
+    out2, ids2, w2 = torch.empty_like(out), torch.empty_like(ids), torch.empty_like(w)
+    N.check(N.load().nsx_moe_forward(C.byref(layer._c), h.data_ptr(), T, out2.data_ptr(), ids2.data_ptr(),
+                                     w2.data_ptr(), narrow.data_ptr(), narrow.numel(), N.stream_ptr(dev)), "forward")
+    assert torch.equal(ids, ids2) and torch.equal(w, w2) and torch.equal(out, out2)
