@@ -200,12 +200,13 @@ def fused_gemv(raw, dtype, x: torch.Tensor, n_rows: int, K: int,
                 if t is not None and (not t.is_cuda or t.dtype != torch.float32 or not t.is_contiguous()
                                       or t.numel() != n):
                     raise ValueError(f"{name} must be a contiguous fp32 device tensor of {n} elements")
-            # several tokens: the activation terms of the matrix-core path (stream-ordered, as y)
+            args = (int(dtype), flat.data_ptr(), n_rows, K, xc.data_ptr(), N.act_dtype_code(xc.dtype), T, y.data_ptr(),
+                    None if bias is None else bias.data_ptr(), None if resid is None else resid.data_ptr())
+            # several tokens: scratch for the activation terms of the matrix-core path (stream-ordered, as y)
             nws = lib.nsx_gemv_workspace_bytes(int(dtype), n_rows, K, T) if T > 1 else 0
-            ws = torch.empty(nws, dtype=torch.uint8, device=x2.device) if nws > 0 else None
-            N.check(lib.nsx_fused_gemv_ws(int(dtype), flat.data_ptr(), n_rows, K, xc.data_ptr(),
-                                          N.act_dtype_code(xc.dtype), T, y.data_ptr(),
-                                          None if bias is None else bias.data_ptr(),
-                                          None if resid is None else resid.data_ptr(),
-                                          None if ws is None else ws.data_ptr(), nws, s), "fused_gemv")
+            if nws > 0:
+                ws = torch.empty(nws, dtype=torch.uint8, device=x2.device)
+                N.check(lib.nsx_fused_gemv_ws(*args, ws.data_ptr(), nws, s), "fused_gemv")
+            else:
+                N.check(lib.nsx_fused_gemv_ex(*args, s), "fused_gemv")
     return y if out_dtype == torch.float32 else y.to(out_dtype)
