@@ -102,7 +102,8 @@ int nsx_fused_gemv_ex(int ggml_type, const void *raw, int64_t n_rows, int64_t K,
                       const float *resid, void *stream);
 /* nsx_fused_gemv_ex with a caller's workspace, in which calls of several tokens
  * keep their activation terms for the matrix cores (products of the exact
- * weight codes and of 33 significant bits of each activation, fp32 sums):
+ * weight codes and of all 24 bits of each activation down to 2^-160 of its
+ * token's largest, fp32 sums):
  * nsx_gemv_workspace_bytes for the same arguments says how much (0: none is
  * used). 16-byte aligned, need not be cleared, free for other use once the
  * call's work on the stream is done; NULL: as nsx_fused_gemv_ex, on the

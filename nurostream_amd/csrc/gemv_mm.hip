@@ -2,11 +2,12 @@
 // cores (nsx_fused_gemv; the reference's compute/triton_kernels.py:199-228
 // fuses one token).
 //
-// y = x . W^T with every weight code exact in f16 and every activation as the
-// sum of three f16 terms of a power-of-two-scaled copy: 33 significant bits,
-// so no more is lost than a product of fp32 values loses, and the matrix
-// cores' sums are fp32. v_mfma_f32_16x16x32_f16 with A = 16 rows of terms x 32
-// elements and B = 32 elements x 16 weight rows. The 16 rows of A are
+// y = x . W^T with every weight code exact in bf16 and every activation as the
+// sum of three bf16 terms of a power-of-two-scaled copy: its 24 bits, whatever
+// the token's other activations are (gm_split says down to where), so the
+// products are those of fp32 values, and the matrix cores' sums are fp32.
+// v_mfma_f32_16x16x32_bf16 with A = 16 rows of terms x 32 elements and B = 32
+// elements x 16 weight rows. The 16 rows of A are
 //   up to 5 tokens:  row j = term j / 5 of token j % 5, one instruction;
 //   up to 8:  row j = term j / 8 of token j % 8, then a second instruction
 //     whose rows j < 8 are term 2;
@@ -24,9 +25,10 @@
 // K is taken in passes over groups of GM_GROUP tiles whose sums wait in LDS.
 //
 // Bound: the weight bytes, then the decode's VALU instructions (about 20 per 8 codes
-// of a lane). Measured, 200000 x 2880, one call: Q8_0 at 8 tokens 144 us (4.3 TB/s) against 1150
-// for the VALU kernel, which decodes a weight per 4 tokens; MXFP4 at 5 tokens 82 / 622; Q4_0 83 /
-// 626; Q4_K 98 / 645; Q6_K 157 / 494.
+// of a lane). Measured, 200000 x 2880, one call: Q8_0 at 8 tokens 146 us (4.2 TB/s) against 1150
+// for the VALU kernel, which decodes a weight per 4 tokens; MXFP4 at 5 tokens 81 / 622; Q4_0 95 /
+// 626; Q4_K 95 / 645; Q6_K 172 / 494. (Terms and codes in f16, whose packed arithmetic decodes with fewer
+// instructions: 142, 81, 82, 97, 155, but a token's small values lost bits beside a large one.)
 #include "gemv_mm.h"
 
 #include <algorithm>
@@ -39,9 +41,8 @@ constexpr int GM_GROUP = 16;   // tiles whose sums wait in LDS between passes ov
 constexpr int GM_PS = 20;      // floats between the A rows of a partial tile (conflict-free writes)
 constexpr int GM_MAXT = 16;
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef short s4 __attribute__((ext_vector_type(4)));  // four bf16 (the 16-element product's operands)
 
 // A format's K unit (the smallest part of a row with scales of its own): elements, bytes.
 template <int FMT> struct Unit { static constexpr int E = 32, B = FMT == NSX_Q8_0 ? 34 : FMT == NSX_Q4_0 ? 18 : 17; };
@@ -49,8 +50,8 @@ template <> struct Unit<NSX_Q4_K> { static constexpr int E = 256, B = 144; };
 template <> struct Unit<NSX_Q6_K> { static constexpr int E = 256, B = 210; };
 
 // Waves of a workgroup: 16 where a sixteenth of K leaves each its 128 registers without spilling, else 8 with 256
-// (200000 x 2880: Q4_0 at 5 tokens 83 us against 99 with 8 waves, at 8 tokens 86 / 101, but at 16 tokens 150 / 106;
-// MXFP4 65536 x 4096 at 5 tokens 41 / 52; Q8_0 117 / 131, at 8 tokens 169 / 144; Q4_K and Q6_K blocks of 256 spill).
+// (200000 x 2880: Q4_0 at 5 tokens 95 us against 104 with 8 waves, at 8 tokens 96 / 103, but at 16 tokens 133 / 111;
+// MXFP4 65536 x 4096 at 5 tokens 40 / 50; Q8_0 120 / 142, at 8 tokens 167 / 146; Q4_K and Q6_K blocks of 256 spill).
 template <int FMT>
 constexpr int gm_waves(int nm) { return Unit<FMT>::E == 32 && nm <= (FMT == NSX_Q8_0 ? 1 : 2) ? 16 : 8; }
 // Elements a wave holds terms for, in 32s: 4 registers per 32 elements and instruction, what the staged pieces leave of
@@ -101,14 +102,32 @@ struct LdsRow {
   }
 };
 
-__device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
-__device__ __forceinline__ uint32_t as_u(h2 v) { return __builtin_bit_cast(uint32_t, v); }
-// two code bytes of w (selected by sel's low bytes) under 0x64: the f16 values 1024 + code
-__device__ __forceinline__ h2 biased(uint32_t w, uint32_t sel) {
-  return as_h2(__builtin_amdgcn_perm(0x64646464u, w, sel));
+// Two bf16 from the halves of two fp32 whose lower halves are zero.
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
 }
-constexpr uint32_t SEL01 = 0x04010400u, SEL23 = 0x04030402u;
-__device__ __forceinline__ h2 both(float v) { return h2{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ float byte_of(uint32_t w, int i) { return (float)((w >> (8 * i)) & 0xFFu); }
+__device__ __forceinline__ float sbyte_of(uint32_t w, int i) { return (float)(int8_t)(w >> (8 * i)); }
+// Four bytes, unsigned or signed, as bf16.
+__device__ __forceinline__ v2u bytes4(uint32_t w) {
+  return v2u{pack2(byte_of(w, 0), byte_of(w, 1)), pack2(byte_of(w, 2), byte_of(w, 3))};
+}
+__device__ __forceinline__ v2u sbytes4(uint32_t w) {
+  return v2u{pack2(sbyte_of(w, 0), sbyte_of(w, 1)), pack2(sbyte_of(w, 2), sbyte_of(w, 3))};
+}
+// Four bytes of 0..15 as bf16: as fp8 (e4m3) such a byte is its value / 512, subnormal or not.
+__device__ __forceinline__ v2u nibbles4(uint32_t w) {
+  return v2u{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 512.f, false)),
+             __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 512.f, true))};
+}
+// Bytes 2 B and 2 B + 1 of e2m1 codes, a byte's low one first, as bf16 times 2.
+template <int B>
+__device__ __forceinline__ v2u fp4x4(uint32_t w) {
+  return v2u{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 2.f, 2 * B)),
+             __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 2.f, 2 * B + 1))};
+}
+// The codes above and below are taken as bytes whose low bits are zero: 2^this times the weight's.
+template <int FMT> constexpr int GM_CODE_EXP = FMT == NSX_Q4_0 ? 4 : FMT == NSX_Q6_K ? 2 : 0;
 
 template <int NM>
 __device__ __forceinline__ int gm_token(int j) { return NM == 1 ? j % 5 : NM == 2 ? j % 8 : j; }
@@ -116,9 +135,9 @@ __device__ __forceinline__ int gm_token(int j) { return NM == 1 ? j % 5 : NM == 
 // ---------------------------------------------------------------------------
 // Activation terms, laid out as the lanes of the product kernel hold them:
 //   per unit and instruction m its operands, [piece][lane][16 B]: a format of 32-element units has one piece; Q4_K
-//   eight (sub-blocks 0..7) and one with the sub-blocks' sums / 32 (lane group 0: elements 0..7; zero elsewhere);
+//   eight (sub-blocks 0..7) and one with the sub-blocks' sums (lane group 0: elements 0..7; zero elsewhere);
 //   Q6_K eight of two 16-element products each;
-//   then 16 exponents: slot j's token was scaled by 2^(its exponent).
+//   then 16 exponents: slot j's sums are 2^(its exponent) times its token's.
 template <int FMT> constexpr int GM_PIECES = FMT == NSX_Q4_K ? 9 : FMT == NSX_Q6_K ? 8 : 1;
 template <int FMT>
 __host__ __device__ constexpr int64_t gm_terms_bytes(int64_t K, int nm) {
@@ -138,19 +157,22 @@ __device__ __forceinline__ int gm_elem(int pc, int g, int v) {
   }
 }
 
-// Terms 0..2 of the scaled activation v: its leading 11 bits, the next 11, the rest; each is exact in f16 (down to
-// f16's subnormals, 2^-39 of the token's largest value). An infinite or NaN v is its own first term.
-__device__ __forceinline__ void gm_split(float v, _Float16 (&t)[3]) {
-  auto top = [](float x) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xFFFFE000u); };
+// Terms 0..2 of the scaled activation v: its leading 8 bits, the next 8, the rest, each exact in bf16. The token's
+// largest finite |x| goes to 2^60 .. 2^61: an activation down to 2^-160 of it keeps all its 24 bits (terms from 2^-126 on
+// are normal), and the sums of a row stay within fp32's range. (One grid of f16 terms for a token would lose a bit for
+// each factor of two below 2^-15 of its largest value: with that value under a zero code, what is left of the row.) An
+// infinite or NaN v is its own first term.
+constexpr int GM_TOP = 61;  // the largest |x| < 2^GM_TOP
+__device__ __forceinline__ void gm_split(float v, uint16_t (&t)[3]) {
+  auto top = [](float x) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & 0xFFFF0000u); };
   const bool fin = fabsf(v) <= 3.4028235e38f;
-  const float hi = fin ? top(v) : v;
-  const float r = fin ? v - hi : 0.f, mid = top(r);
-  t[0] = (_Float16)hi;
-  t[1] = (_Float16)mid;
-  t[2] = (_Float16)(r - mid);
+  const float hi = top(v), r = fin ? v - hi : 0.f, mid = top(r), lo = r - mid;
+  t[0] = (uint16_t)((__builtin_bit_cast(uint32_t, v) >> 16) | (v != v ? 0x40u : 0u));  // (a NaN stays one)
+  t[1] = (uint16_t)(__builtin_bit_cast(uint32_t, mid) >> 16);
+  t[2] = (uint16_t)(__builtin_bit_cast(uint32_t, lo) >> 16);
 }
 
-// Workgroup (token, part of K): the token's scale (its largest finite |x| goes to 2^14 .. 2^15) from the whole row,
+// Workgroup (token, part of K): the token's scale from the whole row,
 // then its slots' terms of the part's units; token 0's workgroups clear the slots that hold no token.
 template <int FMT, int NM>
 __global__ __launch_bounds__(256) void gm_terms_kernel(const void* __restrict__ x, int dt, int K, int T,
@@ -171,27 +193,27 @@ __global__ __launch_bounds__(256) void gm_terms_kernel(const void* __restrict__ 
   if ((tid & 63) == 0) part[tid >> 6] = mx;
   __syncthreads();
   mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-  int ex = 15;
+  int ex = GM_TOP;
   if (mx > 0.f) (void)frexpf(mx, &ex);  // mx < 2^ex
-  const int e = 15 - ex;
+  const int e = GM_TOP - ex;
   int32_t* exps = (int32_t*)(ws + gm_terms_bytes<FMT>(K, NM));
-  auto store = [&](int slot, int m, int u, int pc, int g, const h8& h) {
-    *(h8*)(ws + ((((int64_t)u * PC + pc) * NM + m) * 64 + 16 * g + slot) * 16) = h;
+  auto store = [&](int slot, int m, int u, int pc, int g, const v4u& h) {
+    *(v4u*)(ws + ((((int64_t)u * PC + pc) * NM + m) * 64 + 16 * g + slot) * 16) = h;
   };
   // run r of 8 elements -> piece pc = r / 4 of lane group g = r % 4 (Q4_K's sums: below)
   const int runs = K / 8, per = (runs + (int)gridDim.y - 1) / (int)gridDim.y;
   const int r1 = min(runs, per * ((int)blockIdx.y + 1));
   for (int r = per * (int)blockIdx.y + tid; r < r1; r += 256) {
     const int u = r / ROWS, pc = (r % ROWS) >> 2, g = r & 3;
-    _Float16 t[8][3];
+    uint16_t t[8][3];
 #pragma unroll
     for (int v = 0; v < 8; ++v)
       gm_split(ldexpf(nsx_load_act(x, dt, x0 + (int64_t)u * UE + gm_elem<FMT>(pc, g, v)), e), t[v]);
 #pragma unroll
     for (int term = 0; term < 3; ++term) {
-      h8 h;
+      v4u h;
 #pragma unroll
-      for (int v = 0; v < 8; ++v) h[v] = t[v][term];
+      for (int v = 0; v < 4; ++v) h[v] = t[2 * v][term] | (uint32_t)t[2 * v + 1][term] << 16;
       if (NM == 1) store(5 * term + tok, 0, u, pc, g, h);
       else if (NM == 2) store(term == 1 ? 8 + tok : tok, term == 2 ? 1 : 0, u, pc, g, h);
       else store(tok, term, u, pc, g, h);
@@ -203,20 +225,20 @@ __global__ __launch_bounds__(256) void gm_terms_kernel(const void* __restrict__ 
     const bool on = (tid >> 3) < pu && u < all;
     float s = 0.f;
     for (int i = 0; i < 32; ++i) s += on ? ldexpf(nsx_load_act(x, dt, x0 + (int64_t)u * UE + 32 * (tid & 7) + i), e) : 0.f;
-    _Float16 t[3];
-    gm_split(s * 0.03125f, t);  // (32 values below 2^15: within f16's range)
+    uint16_t t[3];
+    gm_split(s, t);
     if (on) {
 #pragma unroll
       for (int term = 0; term < 3; ++term) {
         const int slot = NM == 1 ? 5 * term + tok : NM == 2 ? (term == 1 ? 8 + tok : tok) : tok;
         const int m = NM == 1 ? 0 : NM == 2 ? (term == 2 ? 1 : 0) : term;
         uint8_t* p = ws + ((((int64_t)u * PC + 8) * NM + m) * 64 + slot) * 16;
-        *(_Float16*)(p + 2 * (tid & 7)) = t[term];
-        for (int g = 1; g < 4; ++g) *(_Float16*)(p + 16 * 16 * g + 2 * (tid & 7)) = (_Float16)0.f;
+        *(uint16_t*)(p + 2 * (tid & 7)) = t[term];
+        for (int g = 1; g < 4; ++g) *(uint16_t*)(p + 16 * 16 * g + 2 * (tid & 7)) = 0;
       }
     }
   }
-  if (blockIdx.y == 0 && tid < 16 && gm_token<NM>(tid) == tok) exps[tid] = e;
+  if (blockIdx.y == 0 && tid < 16 && gm_token<NM>(tid) == tok) exps[tid] = e + GM_CODE_EXP<FMT>;
   if (tok == 0) {  // slots without a token (NM 2: the second instruction has 8 more)
     const int all = K / UE * PC;
     for (int i = (int)blockIdx.y * 256 + tid; i < all * NM * 64; i += 256 * (int)gridDim.y) {
@@ -247,23 +269,22 @@ struct GmArgs {
 // The terms of one unit in registers.
 template <int FMT, int NM>
 struct Terms {
-  h8 a[GM_PIECES<FMT>][NM];
+  b8 a[GM_PIECES<FMT>][NM];
 };
 
-__device__ __forceinline__ h8 gm_h8(h2 a, h2 b, h2 c, h2 d) {
-  return __builtin_bit_cast(h8, v4u{as_u(a), as_u(b), as_u(c), as_u(d)});
-}
+__device__ __forceinline__ b8 gm_b8(v2u a, v2u b) { return __builtin_bit_cast(b8, v4u{a.x, a.y, b.x, b.y}); }
 
 template <int N>
-__device__ __forceinline__ v4f gm_mfma(const h8 (&x)[N], h8 w, v4f c) {
+__device__ __forceinline__ v4f gm_mfma(const b8 (&x)[N], b8 w, v4f c) {
 #pragma unroll
-  for (int m = 0; m < N; ++m) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[m], w, c, 0, 0, 0);
+  for (int m = 0; m < N; ++m) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[m], w, c, 0, 0, 0);
   return c;
 }
 
 // y += unit (its bytes from o on in this lane's weight row) times the terms. MXFP4: times the tokens' scales as well (te, the
 // A rows' scale exponents): a block scale alone may lie far outside the range of the product. The other formats' scales
-// are f16, so the sums cannot leave fp32's range and the tokens' scales wait for the end.
+// are f16, so the sums cannot leave fp32's range and the tokens' scales wait for the end. bf16 holds every code, a zero
+// weight's as zero, but not Q4_K's with its sub-block's scale: those multiply the sums. (A block whose scale is infinite makes its row NaN: the terms' sums meet behind it.)
 template <int FMT, int NM>
 __device__ __forceinline__ void gm_unit(const LdsRow& R, const LdsRow& S0, int o, const Terms<FMT, NM>& X, int g, const int (&te)[4], v4f& y) {
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
@@ -273,48 +294,35 @@ __device__ __forceinline__ void gm_unit(const LdsRow& R, const LdsRow& S0, int o
   };
   if constexpr (FMT == NSX_Q8_0) {
     const v2u w = R.words(o + 2);
-    const h2 off = both(-1152.f);
-    const uint32_t w0 = w.x ^ 0x80808080u, w1 = w.y ^ 0x80808080u;
-    const h8 b = gm_h8(biased(w0, SEL01) + off, biased(w0, SEL23) + off, biased(w1, SEL01) + off, biased(w1, SEL23) + off);
-    add(gm_mfma(X.a[0], b, zero), nsx_h2f(R.get<uint16_t>(o)));
-  } else if constexpr (FMT == NSX_Q4_0) {
-    const uint32_t w = R.word(o + 2), lo = w & 0x0F0F0F0Fu, hi = w & 0xF0F0F0F0u;
-    const h2 off = both(-1032.f), s16 = both(0.0625f), off16 = both(-72.f);
-    const h8 b = gm_h8(biased(lo, SEL01) + off, biased(lo, SEL23) + off,
-                       __builtin_elementwise_fma(biased(hi, SEL01), s16, off16),
-                       __builtin_elementwise_fma(biased(hi, SEL23), s16, off16));
-    add(gm_mfma(X.a[0], b, zero), nsx_h2f(R.get<uint16_t>(o)));
+    add(gm_mfma(X.a[0], gm_b8(sbytes4(w.x), sbytes4(w.y)), zero), nsx_h2f(R.get<uint16_t>(o)));
+  } else if constexpr (FMT == NSX_Q4_0) {  // q - 8 as the upper half of a signed byte
+    const uint32_t w = R.word(o + 2), lo = ((w << 4) & 0xF0F0F0F0u) ^ 0x80808080u, hi = (w & 0xF0F0F0F0u) ^ 0x80808080u;
+    add(gm_mfma(X.a[0], gm_b8(sbytes4(lo), sbytes4(hi)), zero), nsx_h2f(R.get<uint16_t>(o)));
   } else if constexpr (FMT == NSX_MXFP4) {
     const uint32_t w = R.word(o + 1);
-    const h8 b = gm_h8(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 1),
-                       __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 2), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 2.0f, 3));
-    add(gm_mfma(X.a[0], b, zero), nsx_mx_scale_half(R.get<uint8_t>(o)));
+    add(gm_mfma(X.a[0], gm_b8(fp4x4<0>(w), fp4x4<1>(w)), zero), nsx_mx_scale_half(R.get<uint8_t>(o)));
   } else if constexpr (FMT == NSX_Q4_K) {
     const v4u H = R.get<v4u>(o);  // d | dmin, scales[12]
     const uint32_t sc03 = H.y & 0x3F3F3F3Fu, sc47 = (H.w & 0x0F0F0F0Fu) | ((H.y >> 2) & 0x30303030u);
     const uint32_t mn03 = H.z & 0x3F3F3F3Fu, mn47 = ((H.w >> 4) & 0x0F0F0F0Fu) | ((H.z >> 2) & 0x30303030u);
-    const h2 k1024 = both(1024.f), km1024 = both(-1024.f), s16 = both(0.0625f), km64 = both(-64.f);
     v4f acc = zero;
+    auto sub = [&](const b8 (&x)[NM], uint32_t q0, uint32_t q1, float sc) {
+      const v4f d = gm_mfma(x, gm_b8(nibbles4(q0), nibbles4(q1)), zero);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = fmaf(sc, d[i], acc[i]);
+    };
 #pragma unroll
     for (int pr = 0; pr < 4; ++pr) {  // sub-blocks 2 pr (low nibbles) and 2 pr + 1 (high ones)
-      const uint32_t scw = pr < 2 ? sc03 : sc47, b0 = 2u * (pr & 1);
-      const h2 ml = biased(scw, 0x04000400u | b0 << 16 | b0) - k1024;  // (sc, sc)
-      const h2 mh = __builtin_elementwise_fma(biased(scw, 0x04000400u | (b0 + 1) << 16 | (b0 + 1)), s16, km64);
-      const h2 cl = ml * km1024, ch = mh * km1024;
+      const uint32_t scw = pr < 2 ? sc03 : sc47;
       const v2u w = R.get<v2u>(o + 16 + 32 * pr + 8 * g);  // (rows of 16-byte pieces, 4-byte aligned: aligned here)
-      const uint32_t l0 = w.x & 0x0F0F0F0Fu, l1 = w.y & 0x0F0F0F0Fu, h0 = w.x & 0xF0F0F0F0u, h1 = w.y & 0xF0F0F0F0u;
-      auto sq = [](uint32_t q, uint32_t sel, h2 m, h2 c) { return __builtin_elementwise_fma(biased(q, sel), m, c); };
-      acc = gm_mfma(X.a[2 * pr], gm_h8(sq(l0, SEL01, ml, cl), sq(l0, SEL23, ml, cl), sq(l1, SEL01, ml, cl), sq(l1, SEL23, ml, cl)), acc);
-      acc = gm_mfma(X.a[2 * pr + 1], gm_h8(sq(h0, SEL01, mh, ch), sq(h0, SEL23, mh, ch), sq(h1, SEL01, mh, ch), sq(h1, SEL23, mh, ch)), acc);
+      sub(X.a[2 * pr], w.x & 0x0F0F0F0Fu, w.y & 0x0F0F0F0Fu, byte_of(scw, 2 * (pr & 1)));
+      sub(X.a[2 * pr + 1], (w.x >> 4) & 0x0F0F0F0Fu, (w.y >> 4) & 0x0F0F0F0Fu, byte_of(scw, 2 * (pr & 1) + 1));
     }
-    const h8 mins = gm_h8(biased(mn03, SEL01) - k1024, biased(mn03, SEL23) - k1024, biased(mn47, SEL01) - k1024,
-                          biased(mn47, SEL23) - k1024);
-    const v4f am = gm_mfma(X.a[8], mins, zero);
+    const v4f am = gm_mfma(X.a[8], gm_b8(bytes4(mn03), bytes4(mn47)), zero);
     add(acc, nsx_h2f(H.x & 0xFFFFu));
-    add(am, -32.f * nsx_h2f(H.x >> 16));
-  } else {  // Q6_K: a scale for every 16 elements, sc (q - 32) takes more than f16's 11 bits: 16-element products
+    add(am, -nsx_h2f(H.x >> 16));
+  } else {  // Q6_K: a scale for every 16 elements; q - 32 as the upper six bits of a signed byte
     v4f acc = zero;
-    const h2 off = both(-1056.f);
     uint32_t scw[4];  // the 16 scales
 #pragma unroll
     for (int i = 0; i < 4; ++i) scw[i] = S0.word(o + 192 + 4 * i);
@@ -325,20 +333,17 @@ __device__ __forceinline__ void gm_unit(const LdsRow& R, const LdsRow& S0, int o
       const uint32_t qh = R.word(o + 128 + 32 * h + 16 * hl);
 #pragma unroll
       for (int L = 0; L < 4; ++L) {
-        const uint32_t nib = ((L & 1 ? qb : qa) >> (4 * (L >> 1))) & 0x0F0F0F0Fu;
-        const uint32_t top = L == 0 ? qh << 4 : L == 1 ? qh << 2 : L == 2 ? qh : qh >> 2;
-        const uint32_t q = nib | (top & 0x30303030u);
-        const v2u bw = {as_u(biased(q, SEL01) + off), as_u(biased(q, SEL23) + off)};
-        const h4 b = __builtin_bit_cast(h4, bw);
+        const uint32_t ql = L & 1 ? qb : qa, low = L < 2 ? ql << 2 : ql >> 2;
+        const uint32_t top = L == 0 ? qh << 6 : L == 1 ? qh << 4 : L == 2 ? qh << 2 : qh;
+        const s4 b = __builtin_bit_cast(s4, sbytes4(((low & 0x3C3C3C3Cu) | (top & 0xC0C0C0C0u)) ^ 0x80808080u));
         v4f d = zero;
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
-          const h8 x = X.a[2 * hh + (L >> 1)][m];
-          const h4 xa = L & 1 ? h4{x[4], x[5], x[6], x[7]} : h4{x[0], x[1], x[2], x[3]};
-          d = __builtin_amdgcn_mfma_f32_16x16x16f16(xa, b, d, 0, 0, 0);
+          const v4u x = __builtin_bit_cast(v4u, X.a[2 * hh + (L >> 1)][m]);
+          const s4 xa = __builtin_bit_cast(s4, L & 1 ? v2u{x.z, x.w} : v2u{x.x, x.y});
+          d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xa, b, d, 0, 0, 0);
         }
-        const int si = 8 * h + hl + 2 * L;
-        const float sc = (float)(int8_t)(scw[si >> 2] >> (8 * (si & 3)));
+        const float sc = sbyte_of(scw[(8 * h + hl + 2 * L) >> 2], (8 * h + hl + 2 * L) & 3);
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[i] = fmaf(sc, d[i], acc[i]);
       }
@@ -444,7 +449,7 @@ __global__ __launch_bounds__(64 * gm_waves<FMT>(NM)) void gemv_mm_kernel(GmArgs 
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
           const v4u t = *(const v4u*)(a.terms + ((((int64_t)(u0 + u) * GM_PIECES<FMT> + pc) * NM + m) * 64 + lane) * 16);
-          X[u].a[pc][m] = __builtin_bit_cast(h8, mine ? t : zero);
+          X[u].a[pc][m] = __builtin_bit_cast(b8, mine ? t : zero);
         }
     }
   };

@@ -233,6 +233,50 @@ def test_fused_gemv_matrix_core_path(dev, fmt, T, rows, K, offset, xdt):
     assert torch.equal(z[2:], y[2:])
 
 
+def _zero_codes(raw, fmt, rows, K):
+    """raw with the weight of every row's element 0 a zero code (value exactly 0 in every format)."""
+    be, bb = OQ.LAYOUT[getattr(OQ, fmt)]
+    b = raw.reshape(rows, K // be, bb)[:, 0]
+    if fmt == "Q8_0":
+        b[:, 2] = 0
+    elif fmt == "Q4_0":
+        b[:, 2] = b[:, 2] & 0xF0 | 8
+    elif fmt == "MXFP4":
+        b[:, 1] &= 0xF0
+    elif fmt == "Q4_K":  # and sub-block 0's minimum
+        b[:, 16] &= 0xF0
+        b[:, 8] &= 0xC0
+    else:
+        b[:, 0] &= 0xF0
+        b[:, 128] = b[:, 128] & 0xFC | 2
+    return raw
+
+
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "MXFP4", "Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T", [3, 8, 16])
+def test_fused_gemv_large_value_under_zero_codes(dev, fmt, T):
+    """A token's largest activation takes no bits from its others: tokens with one value 2^24 to 2^120 times the rest
+    under a zero code, so that it adds nothing to any row, against float64. Each row is a sum of fp32 products in
+    fp32: n roundings of 2^-24 of the sum of their sizes at most, in practice their root; 64 (K = 4096) covers it and
+    the reference's own fp32 weights."""
+    from nurostream_amd import _native as N
+    from nurostream_amd.compute.kernels import fused_gemv
+    from nurostream_amd.compute.quant import dequantize
+    rows, K = 6151, 4096
+    t = getattr(OQ, fmt)
+    assert N.load().nsx_gemv_workspace_bytes(t, rows, K, T) > 0
+    w = torch.from_numpy(_zero_codes(_gemv_case(fmt, rows, K, seed=T), fmt, rows, K)).to(dev)
+    x = torch.randn(T, K, generator=torch.Generator().manual_seed(T)).to(dev)
+    for i, p in enumerate((24, 44, 120)):
+        x[i, 0] = 2.0 ** p * 1.375
+    W = dequantize(w, t, rows * K, torch.float32).reshape(rows, K).double()
+    assert bool((W[:, 0] == 0).all())
+    y = fused_gemv(w, t, x, rows, K, out_dtype=torch.float32).double()
+    for i in range(T):
+        ref, size = (W * x[i].double()).sum(1), (W.abs() * x[i].double().abs()).sum(1)
+        assert float(((y[i] - ref).abs() / size).max()) < 64 * 2.0 ** -24, i
+
+
 @pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
 def test_fused_gemv_half_activations(dev, xdt):
     from nurostream_amd.compute.kernels import fused_gemv
