@@ -33,6 +33,9 @@ constexpr int ATTN_MAX_REP = 16;  // query heads per kv head (columns of the mat
 // kernel's lanes hold, and none shorter than a tile per wave.
 constexpr int ATTN_MAX_SPLIT = 128;
 constexpr int ATTN_GRID = 512;
+// A running maximum's start. Finite, not -infinity: keys that all score -infinity (overflowed scores) then get weight
+// e^-infinity = 0 beside it, where the difference of two infinities would make the head NaN.
+constexpr float ATTN_LOWEST = -3.4028235e38f;
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(
   v4f qr[ATTN_D / 16];  // query head i16 (heads past n_rep repeat the last and are not stored)
 #pragma unroll
   for (int j = 0; j < ATTN_D / 16; ++j) qr[j] = *(const v4f*)&qs[min(i16, n_rep - 1)][16 * j + 4 * kq];
-  float m = -INFINITY, l = 0.f;
+  float m = ATTN_LOWEST, l = 0.f;
   v4f acc[4] = {};
   auto step = [&](int tile, AttnTile& cur) {
     const int r0 = tile * ATTN_TILE;
@@ -295,8 +298,8 @@ __global__ __launch_bounds__(64 * NW) void attn_split_kernel(
       mx = fmaxf(mx, s[r]);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    const float mn = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));  // finite: a tile holds a key
-    const float corr = expf(m - mn);                                // 0 on the first tile (m = -inf)
+    const float mn = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
+    const float corr = expf(m - mn);  // (first tile: of nothing)
     m = mn;
     float ls = 0.f;
 #pragma unroll

@@ -4,6 +4,8 @@ embedding row gather, and a whole tiny GPT-OSS model (GGUF on disk) through
 NeuroStream -- eager forward, generate() and the one-graph decode token."""
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -148,6 +150,46 @@ def test_attention_split_edges(dev, heads, window):
         # practice the root of that count; the outputs average such errors over the keys
         assert rel_max(to_np(out), ref.numpy()) < 2e-5, p
         assert torch.equal(kv.v[0][:, p].cpu(), qkv.cpu().reshape(-1, 64)[H + G:])
+
+
+@pytest.mark.parametrize("window", [0, 100, 1000])
+@pytest.mark.parametrize("sink", [True, False])
+def test_attention_keys_of_minus_infinity(dev, window, sink):
+    """Keys whose scores overflow to -infinity have no weight, also where they are a whole tile (16 keys), a wave's
+    tiles, a split or every key but the token's own: against the attention over the other keys in float64."""
+    from nurostream_amd.model.decode import DeviceKV, attn_decode, attn_decode_qkv
+    c = _cfg(n_head=8, n_kv=2, window=window)
+    H, G, R, ctx = c.n_head, c.n_head_kv, c.n_rep, 5000
+    g = torch.Generator().manual_seed(7)
+    kv = DeviceKV(1, c, ctx, dev)
+    K, V = (torch.randn(G, ctx, 64, generator=g) for _ in range(2))
+    K[:, :, 0] = 0
+    sinks = torch.randn(H, generator=g).to(dev) if sink else None
+    still = torch.zeros(32, device=dev)  # no rotation: the first dimension stays the one that overflows
+    for p, dead in ((16, 16), (40, 16), (130, 64), (130, 130), (999, 512), (4999, 4096), (4999, 4999)):
+        qkv = torch.randn(H + 2 * G, 64, generator=g)
+        qkv[:H, 0] = 1e20
+        qkv[H:H + G, 0] = 0
+        Kp = K.clone()
+        Kp[:, p - dead:p, 0] = -1e20  # the keys before the token's own: a product of -1e40
+        if p == 40:
+            Kp = K.clone()
+            Kp[:, :dead, 0] = -1e20  # the first ones
+        Kp[:, p], V[:, p] = qkv[H:H + G], qkv[H + G:]
+        kv.k[0].copy_(Kp)
+        kv.v[0].copy_(V)
+        kv.pos.fill_(p)
+        first = max(0, p + 1 - window) if window else 0
+        live = [j for j in range(first, p + 1) if not bool(Kp[0, j, 0] < 0)]
+        s = (qkv[:H].double().reshape(G, R, 1, 64) * Kp[:, live].double()[:, None]).sum(-1) / 8.0
+        z = sinks.cpu().double().reshape(G, R, 1) if sink else torch.full((G, R, 1), -math.inf, dtype=torch.float64)
+        w = torch.softmax(torch.cat([s, z], -1), -1)[..., :-1]
+        ref = (w[..., None] * V[:, live].double()[:, None]).sum(2).reshape(H, 64).numpy()
+        out = attn_decode(qkv[:H].reshape(-1).to(dev), kv, 0, sinks, window, c)
+        assert rel_max(to_np(out), ref) < 2e-5, (p, dead)  # as for any keys
+        kv.k[0][:, p], kv.v[0][:, p] = 0, 0
+        fused = attn_decode_qkv(qkv.reshape(-1).to(dev), None, None, None, c, still, 1.0, kv, 0, sinks, window)
+        assert torch.equal(fused, out), (p, dead)
 
 
 def test_attention_position_outside_cache_writes_nothing(dev):
