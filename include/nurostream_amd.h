@@ -201,6 +201,10 @@ int64_t nsx_moe_workspace_bytes(const nsx_moe_layer *L, int64_t T);
  * nsx_moe_forward and nsx_moe_forward_addnorm run where the workspace holds
  * one (otherwise passes of 4096; each reads every active expert once). */
 int64_t nsx_moe_workspace_bytes_wide(const nsx_moe_layer *L, int64_t T);
+/* 1 where calls of T tokens run the kernels with work items of up to 64 tokens
+ * (enough tokens per expert and enough items for the chip), 0 where not, -1
+ * for a bad layer. Which runs does not change a result's bits. */
+int nsx_moe_prompt_kernels(const nsx_moe_layer *L, int64_t T);
 
 /* out: (T, n_embd) fp32 = sum over the token's experts, in ascending expert
  * id, of weight * expert_ffn(h). ids/weights: (T, top_k) outputs. */

@@ -3888,15 +3888,23 @@ struct MoePlan {
 // matrix cores, whose lead grows with the tokens per expert
 constexpr int GRP_AUTO_MIN_T = 3;
 constexpr int MQ_AUTO_MIN_PAIRS = 104;
-// Q4_K on the matrix cores takes the 64-token items from this many pairs per expert on (top-8 of 128, 16-token items /
-// these: 4096 x 1536 at T = 64 442 / 465 us, 96 526 / 481, 128 587 / 485, 1024 2617 / 1300; 2048 x 768 at T = 64
-// 153 / 161, 96 176 / 164, 1024 805 / 432).
-constexpr int QG_MIN_PER_EXPERT = 5;
-// MXFP4 takes moe_mx_gemm_kernel from this many pairs per expert on: below, an item's tokens no longer cover the reads of
-// its weights, chunk by chunk (whole layer, us, the kernels above / these, 2880 x 2880, top-4: 128 experts, T = 512 (16
-// pairs per expert) 504 / 514, 1024 753 / 724, 2048 1246 / 1141; 32 experts, T = 128 158 / 185, 256 233 / 243, 512
-// 378 / 357, 1024 612 / 579, 2048 1151 / 1014).
-constexpr int XG_MIN_PER_EXPERT = 48;
+// The prompt kernels (items of up to 64 tokens) need two things: tokens to fill an item, and items to fill the chip,
+// since a workgroup walks all of K for its rows where the kernels with 16-token items cut the work finer.
+// Q4_K (moe_q4k_gemm_kernel; whole layer, us, 16-token items / these). Pairs per expert: 128 experts, top-8, 4096 x
+// 1536, at 4 / 5 / 6 / 8 / 64 of them 420 / 451, 456 / 456, 509 / 458, 564 / 464, 2626 / 1284; 2048 x 768 145 / 154,
+// 160 / 156, 169 / 158, 187 / 160, 804 / 432; 96 experts at 5 / 6 116 / 126, 128 / 130; 32 experts, top-4, 4096 x 1536
+// at 5 154 / 152, 2048 x 768 68 / 59; 10 experts at 12 / 16 / 32 108 / 127, 127 / 128, 189 / 168. Gate/up workgroups:
+// 16 experts, 2048 x 768, 96 of them: at 8 pairs per expert 51 / 56, at 32 89 / 87, 144 at 64: 139 / 109; 2048 x 1024,
+// 128 of them: at 8 52 / 58, at 12 76 / 72; 4096 x 1536, 192: at 8 106 / 84; 8 experts, 1024 x 512, 48: 56 / 74.
+static int qg_min_pairs(int E) { return E < 16 ? 16 : E < 64 ? 5 : 6; }  // per expert
+constexpr int QG_MIN_WGS = 128, QG_MIN_WGS_FEW = 160;                    // (from 12 pairs per expert on; below)
+// MXFP4 (moe_mx_gemm_kernel; the same, the kernels that split K / these). Pairs per expert: 128 experts, top-4, 2880 x
+// 2880, at 8 / 12 / 16 / 32 / 64 of them 376 / 388, 428 / 418, 481 / 455, 686 / 625, 1223 / 1084; 64 experts at 12 / 16
+// 231 / 235, 272 / 251. Down workgroups (the fewer; two a CU are resident): 24 experts, 432 of them, at 64 288 / 306,
+// 720 at 128 498 / 471; 32 experts, 480 at 48, 289 / 275; 20 experts, 360 at 64, 260 / 292, 600 at 128, 425 / 381;
+// 16 experts, 240 at 48, 172 / 188; 4 experts, 115 at 48, 74 / 165.
+constexpr int XG_MIN_PER_EXPERT = 16;
+constexpr int XG_MIN_WGS = 448;
 
 // The Q4_K kernels take K <= 4096 and 16-byte aligned expert rows.
 static bool q4k_fast(const nsx_moe_layer* L) {
@@ -3927,14 +3935,29 @@ static int64_t grp_chunk_tokens(const nsx_moe_layer* L, bool wide = false) {
   return (wide ? GRP_WIDE_PAIRS : GRP_MAX_PAIRS) / std::max(1, (int)L->top_k);
 }
 
+// 64-token items of P pairs, about: one for each active expert while they are less than half full
+static int64_t prompt_items(int E, int64_t P) {
+  return std::max(std::min<int64_t>(E, P), P / GRP_GU_T + E / 2);
+}
+
+static bool qg_pays(const nsx_moe_layer* L, int64_t P) {
+  const int64_t E = L->n_expert, wgs = prompt_items(L->n_expert, P) * (2 * L->n_ff / QG_ROWS);
+  return P >= qg_min_pairs(L->n_expert) * E && wgs >= (P < 12 * E ? QG_MIN_WGS_FEW : QG_MIN_WGS);
+}
+
+static bool xg_pays(const nsx_moe_layer* L, int64_t P) {
+  return P >= XG_MIN_PER_EXPERT * (int64_t)L->n_expert &&
+         prompt_items(L->n_expert, P) * nsx_cdiv(nsx_cdiv(L->n_embd, 64), XG_WAVES) >= XG_MIN_WGS;
+}
+
 static MoePlan moe_plan(const nsx_moe_layer* L, int64_t T, bool wide = false) {
   MoePlan p{};
   p.grouped = use_grouped(L, T);
   p.mq = use_mq(L, T);
   if (p.grouped) T = std::min(T, grp_chunk_tokens(L, wide));
   const int64_t P = T * L->top_k;
-  p.qg = p.mq && P >= QG_MIN_PER_EXPERT * L->n_expert;
-  p.xg = p.grouped && L->layout == NSX_LAYOUT_T64 && P >= XG_MIN_PER_EXPERT * L->n_expert;
+  p.qg = p.mq && qg_pays(L, P);
+  p.xg = p.grouped && L->layout == NSX_LAYOUT_T64 && xg_pays(L, P);
   const bool t64 = L->layout == NSX_LAYOUT_T64;
   p.ggu = mx_geom(L->n_ff, L->n_embd);
   p.gdn = mx_geom(L->n_embd, L->n_ff);
@@ -3989,6 +4012,12 @@ extern "C" int64_t nsx_moe_workspace_bytes(const nsx_moe_layer* L, int64_t T) {
 extern "C" int64_t nsx_moe_workspace_bytes_wide(const nsx_moe_layer* L, int64_t T) {
   if (check_layer(L, T) != NSX_OK) return -1;
   return moe_plan(L, T, true).total;
+}
+
+extern "C" int nsx_moe_prompt_kernels(const nsx_moe_layer* L, int64_t T) {
+  if (check_layer(L, T) != NSX_OK) return -1;
+  const MoePlan p = moe_plan(L, T, true);
+  return p.qg || p.xg;
 }
 
 // tokens per pass of a grouped call of T tokens: wide ones where the workspace holds such a pass

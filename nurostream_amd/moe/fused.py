@@ -128,6 +128,10 @@ class MoELayer:
             self._ws[T] = ws
         return ws
 
+    def prompt_kernels(self, T: int) -> bool:
+        """Whether T tokens run the kernels with work items of up to 64 tokens."""
+        return N.load().nsx_moe_prompt_kernels(C.byref(self._c), T) == 1
+
     def _check_buffers(self, T: int, out: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor) -> None:
         """The native call writes through raw pointers: each output must be a
         contiguous tensor of exactly the expected shape and dtype on this

@@ -108,6 +108,34 @@ def test_workspace_bytes_by_dispatch(lib):
     assert lib.nsx_moe_workspace_bytes(C.byref(L), 8) < 0
 
 
+@pytest.mark.parametrize("fmt,n_expert,top_k,n_embd,n_ff,pairs,want", [
+    # MXFP4 (kernels that split K / prompt kernels, us, at these sizes on one MI355X): 376 / 388, 481 / 455, 686 / 625
+    ("MXFP4", 128, 4, 2880, 2880, 8, 0), ("MXFP4", 128, 4, 2880, 2880, 16, 1), ("MXFP4", 128, 4, 2880, 2880, 32, 1),
+    # 272 / 251, 289 / 275, 228 / 216 (few items: the older kernels)
+    ("MXFP4", 64, 4, 2880, 2880, 16, 1), ("MXFP4", 32, 4, 2880, 2880, 48, 1), ("MXFP4", 32, 4, 2880, 2880, 32, 0),
+    # few experts: 172 / 188, 119 / 169, 88 / 144, 74 / 165, 60 / 96, 288 / 306, 260 / 292
+    ("MXFP4", 16, 4, 2880, 2880, 48, 0), ("MXFP4", 8, 2, 2880, 2880, 48, 0), ("MXFP4", 8, 2, 2880, 1440, 48, 0),
+    ("MXFP4", 4, 2, 2880, 2880, 48, 0), ("MXFP4", 8, 4, 1024, 1024, 48, 0), ("MXFP4", 24, 4, 2880, 2880, 64, 0),
+    ("MXFP4", 20, 4, 2880, 2880, 64, 0),
+    # Q4_K: 420 / 451, 509 / 458, 154 / 152, 408 / 248
+    ("Q4_K", 128, 8, 4096, 1536, 4, 0), ("Q4_K", 128, 8, 4096, 1536, 6, 1), ("Q4_K", 32, 4, 4096, 1536, 5, 1),
+    ("Q4_K", 8, 2, 4096, 3584, 64, 1),
+    # 51 / 56, 52 / 58, 83 / 103, 56 / 74, 108 / 127
+    ("Q4_K", 16, 4, 2048, 768, 8, 0), ("Q4_K", 16, 4, 2048, 1024, 8, 0), ("Q4_K", 8, 8, 2048, 768, 64, 0),
+    ("Q4_K", 8, 2, 1024, 512, 64, 0), ("Q4_K", 10, 2, 2048, 4096, 12, 0)])
+def test_prompt_kernels_where_they_are_faster(lib, fmt, n_expert, top_k, n_embd, n_ff, pairs, want):
+    """The rule that takes a call to the kernels with 64-token items, at measured points (pairs per expert)."""
+    L = _gptoss_layer()
+    L.n_expert, L.top_k, L.n_embd, L.n_ff = n_expert, top_k, n_embd, n_ff
+    L.gate_base = L.up_base = L.down_base = 1 << 20
+    L.gate_stride = L.up_stride = L.down_stride = 1 << 24
+    if fmt == "Q4_K":
+        L.ggml_type, L.layout, L.dispatch = int(GGMLType.Q4_K), N.LAYOUT_GGUF, N.DISPATCH_MFMA
+    assert lib.nsx_moe_prompt_kernels(C.byref(L), pairs * n_expert // top_k) == want
+    L.top_k = 0
+    assert lib.nsx_moe_prompt_kernels(C.byref(L), 8) == -1
+
+
 def test_validation_errors_return_codes(lib):
     # unsupported block type: NotImplemented, with a message
     rc = lib.nsx_dequantize(13, None, 176, 256, None, N.DT_F32, None)  # Q5_K

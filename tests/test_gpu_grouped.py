@@ -261,16 +261,18 @@ def test_config4_qwen3_t32_mfma(config4_t32):
     _check_all_tokens(cfg, t, h, im, wm, om, 1e-5, oracle=c["oracle"])
 
 
-@pytest.mark.parametrize("n_embd,n_ff,T,bias", [(512, 256, 300, False), (512, 768, 41, True), (1024, 512, 1100, False)])
+@pytest.mark.parametrize("n_embd,n_ff,T,bias", [(512, 256, 300, False), (512, 768, 41, True), (1024, 512, 1100, False),
+                                               (512, 256, 1030, True), (512, 2816, 41, True), (256, 2816, 27, False)])
 def test_mfma_q4k_large_batches_equal_small_ones(dev, n_embd, n_ff, T, bias):
-    """Q4_K with at least 5 pairs per expert runs 64-token items (one to four token tiles, experts of
-    several items, an odd number of super-blocks, more pairs than one sort takes); slices of at most 7
-    tokens (56 pairs of 12 experts) run the 16-token items. Each (pair, row) is the same sequence of
+    """Q4_K with many pairs per expert and enough work items runs 64-token items (one to four token tiles, experts of
+    several items, an odd number of super-blocks, more pairs than one sort takes; the first two are too few for them:
+    16-token items, of 300 and 41 tokens); slices of at most 7 tokens (56 pairs of 12 experts) run the 16-token items. Each (pair, row) is the same sequence of
     operations: identical outputs."""
     from nurostream_amd import synth
     cfg = synth.MoEConfig("q4k", synth.GGMLType.Q4_K, 12, 8, n_embd, n_ff, "qwen3", "silu_mul", bias, torch.float32)
     t = synth.make_layer(cfg, seed=29, device=dev)
     layer = _layer(cfg, t, "gguf", dispatch="mfma")
+    assert layer.prompt_kernels(T) == ((n_ff, T) not in ((256, 300), (768, 41))) and not layer.prompt_kernels(7)
     h = synth.activations(T, n_embd, seed=T, device=dev) * torch.linspace(0.01, 30, T, device=dev)[:, None]
     out, ids, wts = layer(h)
     for t0 in [*range(0, min(T, 84), 7), T // 2, T - 7]:
@@ -282,6 +284,23 @@ def test_mfma_q4k_large_batches_equal_small_ones(dev, n_embd, n_ff, T, bias):
         torch.testing.assert_close(out[t0:t0 + n][same], o[same], rtol=0, atol=2e-6 * float(o.abs().max()))
     ref, _, _, _ = _oracle_layer(cfg, t, h[:40].cpu().numpy())
     assert rel_max(to_np(out[:40]), ref) < 1e-5
+
+
+@pytest.mark.parametrize("n_embd,n_ff", [(512, 2816), (768, 4096)])
+def test_q4k_prompt_kernel_bitwise(dev, n_embd, n_ff):
+    """64-token items (63 tokens for each of 8 experts) against 16-token ones, bit for bit: a router that gives every
+    token the same experts and weights in any batch."""
+    from nurostream_amd import synth
+    cfg = synth.MoEConfig("q4k", synth.GGMLType.Q4_K, 12, 8, n_embd, n_ff, "qwen3", "silu_mul", False, torch.float32)
+    t = synth.make_layer(cfg, seed=37, device=dev)
+    t["router_w"] = torch.zeros_like(t["router_w"])
+    layer = _layer(cfg, t, "gguf", dispatch="mfma")
+    assert layer.prompt_kernels(63) and not layer.prompt_kernels(7)
+    h = synth.activations(63, n_embd, seed=2, device=dev)
+    out, _, _ = layer(h)
+    for t0 in range(0, 63, 7):
+        o, _, _ = layer(h[t0:t0 + 7])
+        assert torch.equal(out[t0:t0 + 7], o), t0
 
 
 def test_q4k_gemm_kernel_bitwise(dev):
@@ -318,6 +337,26 @@ def test_mx_gemm_kernel_bitwise(dev, n_embd, n_ff, T, bias, slabs):
     og, ig, _ = lg(h)
     n = torch.bincount(ig.flatten().long(), minlength=8)
     assert n.sum() >= 48 * 8 and n.max() > 64  # (the rule's 48 pairs per expert; a second work item)
+    assert torch.equal(ip, ig) and torch.equal(op, og)
+
+
+@pytest.mark.parametrize("n_embd,n_ff,T,bias,slabs", [(864, 96, 2048, False, False),   # partial K-steps and row tiles
+                                                     (864, 64, 1900, True, True),     # one tile of gate and up
+                                                     (2080, 224, 1000, True, False),  # a unit of one tile
+                                                     (896, 2880, 1850, True, False)])  # six steps a down chunk, then five
+def test_mx_prompt_kernel_bitwise(dev, n_embd, n_ff, T, bias, slabs):
+    """The kernels with 64-token items at sizes that run them (few experts of many items), bit for bit the per-pair
+    ones."""
+    from nurostream_amd import synth
+    cfg = synth.MoEConfig("mx", synth.GGMLType.MXFP4, 8, 4, n_embd, n_ff, "gptoss",
+                          "clamped_swiglu" if bias else "silu_mul", bias, torch.bfloat16)
+    t = synth.make_layer(cfg, seed=19, device=dev)
+    t["router_b"] = torch.tensor([0.0, 0.3, -0.3, 0.0] * 2, device=dev)
+    lp, lg = (_layer(cfg, t, "t64", slabs=slabs, dispatch=d) for d in ("pairs", "grouped"))
+    assert lg.prompt_kernels(T) and not lp.prompt_kernels(T)
+    h = synth.activations(T, n_embd, seed=T, device=dev)
+    op, ip, _ = lp(h)
+    og, ig, _ = lg(h)
     assert torch.equal(ip, ig) and torch.equal(op, og)
 
 
