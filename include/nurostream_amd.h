@@ -107,8 +107,11 @@ int nsx_fused_gemv_ex(int ggml_type, const void *raw, int64_t n_rows, int64_t K,
  * nsx_gemv_workspace_bytes for the same arguments says how much (0: none is
  * used). 16-byte aligned, need not be cleared, free for other use once the
  * call's work on the stream is done; NULL: as nsx_fused_gemv_ex, on the
- * VALU. No reference counterpart (the reference fuses one token). */
+ * VALU. nsx_gemv_uses_workspace: 1 where the call runs on the matrix cores,
+ * 0 where the VALU is the faster (the workspace then stays unused and may be
+ * NULL). No reference counterpart (the reference fuses one token). */
 int64_t nsx_gemv_workspace_bytes(int ggml_type, int64_t n_rows, int64_t K, int64_t T);
+int nsx_gemv_uses_workspace(int ggml_type, int64_t n_rows, int64_t K, int64_t T);
 int nsx_fused_gemv_ws(int ggml_type, const void *raw, int64_t n_rows, int64_t K,
                       const void *x, int x_dtype, int64_t T, float *y, const float *bias,
                       const float *resid, void *workspace, int64_t workspace_bytes, void *stream);

@@ -64,6 +64,7 @@ _SIGS = {
     "nsx_fused_gemv": (_i, [_i, _p, _i64, _i64, _p, _i, _i64, _p, _p]),
     "nsx_fused_gemv_ex": (_i, [_i, _p, _i64, _i64, _p, _i, _i64, _p, _p, _p, _p]),
     "nsx_gemv_workspace_bytes": (_i64, [_i, _i64, _i64, _i64]),
+    "nsx_gemv_uses_workspace": (_i, [_i, _i64, _i64, _i64]),
     "nsx_fused_gemv_ws": (_i, [_i, _p, _i64, _i64, _p, _i, _i64, _p, _p, _p, _p, _i64, _p]),
     "nsx_fused_gemv_norm": (_i, [_i, _p, _i64, _i64, _p, _p, _p, C.c_float, _p, _p, _p, _p, _p]),
     "nsx_t64_bytes": (_i64, [_i, _i64, _i64]),

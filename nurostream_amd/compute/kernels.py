@@ -203,7 +203,9 @@ def fused_gemv(raw, dtype, x: torch.Tensor, n_rows: int, K: int,
             args = (int(dtype), flat.data_ptr(), n_rows, K, xc.data_ptr(), N.act_dtype_code(xc.dtype), T, y.data_ptr(),
                     None if bias is None else bias.data_ptr(), None if resid is None else resid.data_ptr())
             # several tokens: scratch for the activation terms of the matrix-core path (stream-ordered, as y)
-            nws = lib.nsx_gemv_workspace_bytes(int(dtype), n_rows, K, T) if T > 1 else 0
+            nws = 0
+            if T > 1 and lib.nsx_gemv_uses_workspace(int(dtype), n_rows, K, T):
+                nws = lib.nsx_gemv_workspace_bytes(int(dtype), n_rows, K, T)
             if nws > 0:
                 ws = torch.empty(nws, dtype=torch.uint8, device=x2.device)
                 N.check(lib.nsx_fused_gemv_ws(*args, ws.data_ptr(), nws, s), "fused_gemv")

@@ -593,13 +593,9 @@ int gm_fmt(const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtyp
 
 int64_t nsx_gemv_mm_workspace(int t, int64_t n_rows, int64_t K, int64_t T) {
   if (T < 2 || T > GM_MAXT || K < 128) return 0;  // (a wave reads at least 4 blocks of 32)
-  // below these sizes the VALU kernel's one launch is the shorter one (us, VALU / here: Q4_0 at 2 tokens 2880 x 2880
-  // 10.3 / 11.0, 5120 x 2880 13.7 / 12.7; at 3 512 x 4096 12.3 / 12.3, 2048 x 4096 17.1 / 11.7; at 5 512 x 4096 18.4 /
-  // 11.5; Q8_0 and MXFP4 cross there too. The K-quants' wider blocks: Q4_K at 2 tokens 5120 x 2816 13.8 / 16.7,
-  // 12288 x 4096 31.8 / 20.9; Q6_K 23.3 / 26.7, 65536 x 4096 91 / 66; at 3 5120 x 2816 16.8 / 20.4, 12288 x 4096 35 / 27)
   const int64_t least = T == 2 ? (t == NSX_Q6_K ? 64ll : t == NSX_Q4_K ? 24ll : 12ll)
                       : T <= 4 ? (t == NSX_Q6_K ? 24ll : 4ll) : 1ll;
-  if (n_rows * K < least << 20) return 0;
+  if (n_rows * K < least << 20) return 0;  // (nothing smaller is faster here)
   int64_t b = 0;
   switch (t) {
     case NSX_MXFP4: b = gm_terms_bytes<NSX_MXFP4>(K, gm_mode(T)); break;
@@ -610,6 +606,46 @@ int64_t nsx_gemv_mm_workspace(int t, int64_t n_rows, int64_t K, int64_t T) {
     default: return 0;
   }
   return b + 64;
+}
+
+// Where this path is the faster one (us in a graph, VALU kernel / here). The VALU kernel's time grows with rows x K, with
+// K x tokens where rows are few (a row's chain of units, once per 4 tokens) and in steps of its workgroups where K is
+// small; this one's starts at its two launches and a tile's way through LDS, longer for the K-quants' wide blocks and for
+// Q8_0 of 6 to 8 tokens (8 waves) outside K of 2048 .. 3072, where one pass of 12 units a wave holds all of it.
+//  2 tokens: rows x K. Q4_0 2880 x 2880 9.2 / 10.4, 5120 x 2880 13.4 / 12.1; Q4_K 5825 x 2816 14.3 / 16.3, 12288 x 4096
+//   31.8 / 20.9; Q6_K 8192 x 8192 38.7 / 35.1, 16384 x 4096 (two blocks a wave spill) 27.0 / 29.9, 32768 x 2048 29 / 23.
+//  3, 4: Q4_0, MXFP4 from 4 Mi weights on (2048 x 2048 11.3 / 9.6); Q8_0 1024 x 4096 10.0 / 12.1, 2048 x 2048 10.6 / 9.6;
+//   Q4_K 4096 x 1024 9.4 / 11.6, 2896 x 2048 13.4 / 13.1, 1448 x 4096 at 3 13.2 / 15.1, 512 x 8192 at 3 21 / 19.5.
+//  5: Q4_0 1024 x 1024 7.6 / 8.5, 2048 x 512 7.3 / 8.1, 512 x 2048 11.0 / 9.4, 4096 x 256 8.9 / 8.0, 1448 x 1024 10 / 8.4;
+//   Q4_K 1024 x 2048 10.0 / 12.6, 728 x 2816 12.0 / 13.5, 512 x 4096 16.1 / 14.7; Q6_K 728 x 2816 11.1 / 14.0.
+//  6 to 8: MXFP4 1024 x 2048 10.1 / 10.7, 4096 x 256 11.7 / 8.1; Q8_0 1024 x 4096 at 6 18.3 / 20.6, at 8 24 / 20.5, 1024 x
+//   2048 at 8 12.7 / 14.4, 1029 x 2880 21.9 / 12.4; Q4_K 2048 x 1024 at 6 12.6 / 13.0, 4096 x 512 10.9 / 11.7, 8192 x 256
+//   15.8 / 12.3; Q6_K 1448 x 1024 7.9 / 9.9, 4096 x 256 11.6 / 8.9.
+//  9 to 16: Q4_K 1024 x 1024 at 9 10.6 / 13.3, at 16 15 / 12; Q6_K the same, 9.7 / 10.9; the others gain from 1 Mi on.
+static bool gm_pays(int t, int64_t n_rows, int64_t K, int64_t T) {
+  const double n = (double)n_rows * K / (1 << 20);
+  const int64_t kt = K * T;
+  if (T == 2) return t != NSX_Q6_K || K <= 2048 || n >= 68;
+  if (T <= 4) {
+    if (t == NSX_Q8_0) return n >= 4.5 || kt >= 15000 || n_rows >= 2048;
+    return t != NSX_Q4_K || n >= 6 || kt >= 24000 || n_rows >= 10000;
+  }
+  if (T > 8) return n >= 1.25 || (t != NSX_Q4_K && t != NSX_Q6_K) || T >= 12 || kt >= 15000 || n_rows >= 2048;
+  switch (t) {
+    case NSX_Q4_K: return n >= 2.25 || kt >= (T == 5 ? 20000 : 26000) || n_rows >= 5500;
+    case NSX_Q6_K: return n >= 2.25 || kt >= 20000 || n_rows >= 2800;
+    case NSX_Q8_0:
+      if (T > 5) return n >= 4.25 || kt >= (K > 2048 && K <= 3072 ? 17000 : 26000) || n_rows >= 2048;
+      break;
+    case NSX_MXFP4:
+      if (T > 5) return n >= 2.25 || kt >= 15000 || n_rows >= 2800;
+      break;
+  }
+  return n >= 1.25 || kt >= (T == 5 ? 10000 : 15000) || n_rows >= 2800;
+}
+
+int nsx_gemv_mm_takes(int t, int64_t n_rows, int64_t K, int64_t T) {
+  return nsx_gemv_mm_workspace(t, n_rows, K, T) > 0 && gm_pays(t, n_rows, K, T);
 }
 
 int nsx_gemv_mm(int t, const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtype, int64_t T, float* y,

@@ -786,6 +786,10 @@ extern "C" int64_t nsx_gemv_workspace_bytes(int t, int64_t n_rows, int64_t K, in
   return nsx_gemv_mm_workspace(t, n_rows, K, T);
 }
 
+extern "C" int nsx_gemv_uses_workspace(int t, int64_t n_rows, int64_t K, int64_t T) {
+  return nsx_gemv_workspace_bytes(t, n_rows, K, T) > 0 && nsx_gemv_mm_takes(t, n_rows, K, T);
+}
+
 extern "C" int nsx_fused_gemv_ws(int t, const void* raw, int64_t n_rows, int64_t K, const void* x, int x_dtype,
                                  int64_t T, float* y, const float* bias, const float* resid, void* workspace,
                                  int64_t workspace_bytes, void* stream) {
@@ -807,7 +811,7 @@ extern "C" int nsx_fused_gemv_ws(int t, const void* raw, int64_t n_rows, int64_t
     const int64_t need = nsx_gemv_mm_workspace(t, n_rows, K, T);
     NSX_REQUIRE(workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0, NSX_EINVAL,
                 "workspace of %lld bytes, need %lld, 16-byte aligned", (long long)workspace_bytes, (long long)need);
-    if (need > 0) return nsx_gemv_mm(t, raw, n_rows, K, x, x_dtype, T, y, bias, resid, workspace, st);
+    if (nsx_gemv_mm_takes(t, n_rows, K, T)) return nsx_gemv_mm(t, raw, n_rows, K, x, x_dtype, T, y, bias, resid, workspace, st);
   }
   // tokens per launch: as many as one workgroup's LDS holds (<= 64 KiB staged)
   int64_t chunk = 16;

@@ -108,6 +108,29 @@ def test_workspace_bytes_by_dispatch(lib):
     assert lib.nsx_moe_workspace_bytes(C.byref(L), 8) < 0
 
 
+@pytest.mark.parametrize("fmt,rows,K,T,want", [
+    # VALU kernel / matrix-core path, us, at these sizes on one MI355X
+    ("Q4_0", 2880, 2880, 2, 0), ("Q4_0", 5120, 2880, 2, 1), ("Q6_K", 16384, 4096, 2, 0), ("Q6_K", 32768, 2048, 2, 1),
+    ("Q8_0", 1024, 4096, 3, 0), ("Q8_0", 2048, 2048, 3, 1), ("MXFP4", 2048, 2048, 3, 1),  # 10.0 / 12.1, 10.6 / 9.6
+    ("Q4_K", 4096, 1024, 3, 0), ("Q4_K", 2048, 2048, 3, 0), ("Q4_K", 2048, 2816, 3, 0),  # 9.4 / 11.6, 11.4 / 12.9
+    ("Q4_K", 512, 8192, 4, 1), ("Q4_K", 4096, 2816, 3, 1),  # 28.0 / 19.2, 19.5 / 14.3
+    ("Q4_0", 2048, 512, 5, 0), ("Q8_0", 2048, 512, 5, 0), ("Q4_0", 1024, 1024, 6, 0),  # 7.3 / 8.1, 8.0 / 8.3, 7.6 / 9.0
+    ("Q4_0", 512, 4096, 5, 1), ("MXFP4", 4096, 256, 6, 1), ("Q4_0", 2048, 1024, 6, 1),  # 17.6 / 10.6, 11.7 / 8.1, 12 / 9
+    ("MXFP4", 2048, 512, 6, 0), ("MXFP4", 1024, 2048, 6, 0), ("MXFP4", 512, 4096, 6, 1),  # 7.6 / 8.3, 10.1 / 10.7, 16 / 13
+    ("Q8_0", 1024, 4096, 6, 0), ("Q8_0", 1024, 2048, 8, 0),  # 18.3 / 20.6, 12.7 / 14.4
+    ("Q8_0", 1024, 4096, 8, 1), ("Q8_0", 1029, 2880, 8, 1), ("Q8_0", 4096, 512, 6, 1),  # 24 / 20.5, 21.9 / 12.4, 13 / 7.8
+    ("Q4_K", 4096, 256, 5, 0), ("Q4_K", 512, 2816, 5, 0), ("Q4_K", 2048, 1024, 6, 0),  # 9.3 / 10.1, 11.4 / 13.1, 12.6 / 13
+    ("Q4_K", 512, 4096, 5, 1), ("Q4_K", 4096, 1024, 6, 1), ("Q4_K", 8192, 256, 5, 1),  # 16.1 / 14.7, 17.4 / 13.4, 16 / 11
+    ("Q6_K", 512, 2816, 6, 0), ("Q6_K", 2048, 512, 6, 0), ("Q6_K", 512, 4096, 6, 1),  # 12.2 / 13.4, 8.4 / 8.9, 16.3 / 14
+    ("Q4_K", 1024, 1024, 9, 0), ("Q6_K", 1024, 1024, 9, 0), ("Q8_0", 1024, 1024, 9, 1), ("Q4_K", 1024, 1024, 16, 1),
+    ("Q4_0", 4096, 4096, 1, 0), ("Q4_0", 4096, 4096, 17, 0), ("Q4_0", 4096, 96, 16, 0), ("Q4_0", 4096, 33, 8, 0)])
+def test_gemv_of_several_tokens_where_it_is_faster(lib, fmt, rows, K, T, want):
+    """The rule that takes a GEMV of several tokens to the matrix cores, at measured points."""
+    t = int(GGMLType[fmt])
+    assert lib.nsx_gemv_uses_workspace(t, rows, K, T) == want
+    assert want == 0 or lib.nsx_gemv_workspace_bytes(t, rows, K, T) > 0
+
+
 @pytest.mark.parametrize("fmt,n_expert,top_k,n_embd,n_ff,pairs,want", [
     # MXFP4 (kernels that split K / prompt kernels, us, at these sizes on one MI355X): 376 / 388, 481 / 455, 686 / 625
     ("MXFP4", 128, 4, 2880, 2880, 8, 0), ("MXFP4", 128, 4, 2880, 2880, 16, 1), ("MXFP4", 128, 4, 2880, 2880, 32, 1),
