@@ -17,7 +17,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libnsx.so"
 SOURCES = ("quant.hip", "gemv_mm.hip", "moe.hip", "attn.hip", "reader.hip")
-HEADERS = ("nsx_common.h", "raw_dot.h", "gemv_mm.h")
+HEADERS = ("nsx_common.h", "raw_dot.h", "gemv_mm.h", "launch_cache.h")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -518,7 +518,7 @@ int gm_launch(GmArgs a, hipStream_t st) {
   const size_t lds = (size_t)W * a.part_bytes + 2 * W * GM_ROWS * GM_PS * sizeof(float) +
                      (a.npass > 1 ? GM_GROUP * 256 * sizeof(float) : 0);
   const void* k = (const void*)gemv_mm_kernel<FMT, NM, MAXU>;
-  if (lds > 64 * 1024) NSX_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  if (int rc = nsx_allow_lds(k, lds)) return rc;
   const int64_t grid = std::min<int64_t>(nsx_cdiv(a.n_rows, GM_ROWS), nsx_resident_workgroups(k, lds, 64 * W));
   hipLaunchKernelGGL((gemv_mm_kernel<FMT, NM, MAXU>), dim3((unsigned)grid), dim3(64 * W), lds, st, a);
   NSX_LAUNCHED();

@@ -4202,7 +4202,7 @@ static MoeDev make_dev(const nsx_moe_layer* L, const MoePlan& p, char* ws, const
 
 template <bool GU>
 static int launch_xg(const MoePlan& p, const MoeDev& d, hipStream_t st) {
-  NSX_HIP(hipFuncSetAttribute((const void*)moe_mx_gemm_kernel<GU>, hipFuncAttributeMaxDynamicSharedMemorySize, XG_LDS));
+  if (int rc = nsx_allow_lds((const void*)moe_mx_gemm_kernel<GU>, XG_LDS)) return rc;
   const int64_t units = nsx_cdiv(GU ? p.ggu.tiles : p.gdn.tiles, GU ? XG_WAVES / 2 : XG_WAVES);
   return nsx_launch(moe_mx_gemm_kernel<GU>, dim3((unsigned)(8 * nsx_cdiv(p.max_gu_items, 8) * units)), dim3(64 * XG_WAVES),
                     (size_t)XG_LDS, st, d);
@@ -4210,8 +4210,7 @@ static int launch_xg(const MoePlan& p, const MoeDev& d, hipStream_t st) {
 
 template <bool GU>
 static int launch_qg(const MoePlan& p, const MoeDev& d, int rows, hipStream_t st) {
-  const void* k = (const void*)moe_q4k_gemm_kernel<GU>;
-  NSX_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * QG_BUF));
+  if (int rc = nsx_allow_lds((const void*)moe_q4k_gemm_kernel<GU>, 2 * QG_BUF)) return rc;
   const unsigned grid = (unsigned)(8 * nsx_cdiv(p.max_gu_items, 8) * (rows / QG_ROWS));
   return nsx_launch(moe_q4k_gemm_kernel<GU>, dim3(grid), dim3(64 * QG_WAVES), (size_t)(2 * QG_BUF), st, d);
 }

@@ -19,6 +19,8 @@ int nsx_fail(int code, const char* fmt, ...);
 // Workgroups of `kernel` (`threads` threads, `lds` dynamic bytes) resident on the current device at once
 // (CUs x blocks per CU), cached per kernel, LDS size and device.
 int nsx_resident_workgroups(const void* kernel, size_t lds, int threads);
+// `kernel` may be launched with `lds` dynamic bytes (above 64 KB the runtime has to be told, once per kernel and device).
+int nsx_allow_lds(const void* kernel, size_t lds);
 
 #define NSX_HIP(call)                                                           \
   do {                                                                          \

@@ -8,6 +8,7 @@
 #include "mx.h"
 #include "raw_dot.h"
 #include "gemv_mm.h"
+#include "launch_cache.h"
 
 #include <algorithm>
 #include <mutex>
@@ -656,27 +657,31 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_raw_kernel(
   }
 }
 
+int nsx_allow_lds(const void* kernel, size_t lds) {
+  static NsxLdsLimits& limits = *new NsxLdsLimits;  // (never destroyed: a thread may still launch while the process ends)
+  if (lds <= 64 * 1024) return NSX_OK;
+  int dev = 0;
+  NSX_HIP(hipGetDevice(&dev));
+  return limits.allow(kernel, dev, lds, [&](size_t n) {
+    NSX_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n));
+    return (int)NSX_OK;
+  });
+}
+
 // Workgroups of `kernel` (`threads` threads, `lds` bytes) resident on the
 // current device at once: CUs x blocks per CU, cached per kernel and LDS size.
 int nsx_resident_workgroups(const void* kernel, size_t lds, int threads) {
-  struct Entry { const void* k; size_t lds; int threads, dev, n; };
-  static std::mutex mu;
-  static Entry cache[64];
-  static int used = 0;
+  static NsxLaunchCache& cache = *new NsxLaunchCache;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-  std::lock_guard<std::mutex> lock(mu);
-  for (int i = 0; i < used; ++i)
-    if (cache[i].k == kernel && cache[i].lds == lds && cache[i].threads == threads && cache[i].dev == dev)
-      return cache[i].n;
-  int cus = 0, per = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-  if (lds > 64 * 1024) (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, lds) != hipSuccess || per <= 0) per = 1;
-  (void)hipGetLastError();
-  const int n = cus * per;
-  if (used < 64) cache[used++] = Entry{kernel, lds, threads, dev, n};
-  return n;
+  return cache.get(kernel, lds, threads, dev, [&] {
+    int cus = 0, per = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    (void)nsx_allow_lds(kernel, lds);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, lds) != hipSuccess || per <= 0) per = 1;
+    (void)hipGetLastError();
+    return cus * per;
+  });
 }
 
 template <int FMT, int NT>

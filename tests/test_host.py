@@ -256,3 +256,47 @@ def test_parse_size_and_api_on_cpu(tmp_path):
         next(ns.generate("hello"))
     with pytest.raises(N.NativeError):
         ns.model._ffn_block(torch.randn(1, 64), 0)
+
+
+def test_launch_caches(tmp_path):
+    """csrc/launch_cache.h, compiled for the host: an answer is asked for once however many kernels and LDS sizes a
+    process uses, from several threads; an LDS limit only grows, and an error is not remembered."""
+    import subprocess
+
+    from nurostream_amd import build
+    src = tmp_path / "t.cpp"
+    src.write_text(r"""
+#include "launch_cache.h"
+#include <atomic>
+#include <thread>
+#include <vector>
+int main() {
+  NsxLaunchCache c;
+  std::atomic<int> asked{0}, bad{0};
+  std::vector<std::thread> t;
+  for (int n = 0; n < 4; ++n)
+    t.emplace_back([&] {
+      for (int round = 0; round < 3; ++round)
+        for (size_t i = 0; i < 1000; ++i)
+          bad += c.get((const void*)(i % 100 + 1), 1024 * (i / 100), 256, 0, [&] { ++asked; return (int)i; }) != (int)i;
+    });
+  for (auto& x : t) x.join();
+  if (bad) return 1;
+  if (asked != 1000) return 2;
+  NsxLdsLimits l;
+  int set = 0;
+  size_t at = 0;
+  auto ok = [&](size_t n) { ++set; at = n; return 0; };
+  const void* k = (const void*)1;
+  if (l.allow(k, 0, 70000, [](size_t) { return -5; }) != -5) return 3;
+  for (size_t n : {70000, 100000, 80000, 100000, 70000})
+    if (l.allow(k, 0, n, ok) != 0) return 4;
+  if (set != 2 || at != 100000) return 5;
+  if (l.allow(k, 1, 70000, ok) || l.allow((const void*)2, 0, 70000, ok) || set != 4) return 6;
+  return 0;
+}
+""")
+    exe = tmp_path / "t"
+    subprocess.run(["g++", "-std=c++17", "-pthread", "-I", str(build.CSRC), "-o", str(exe), str(src)], check=True,
+                   timeout=100)
+    assert subprocess.run([str(exe)], timeout=60).returncode == 0
