@@ -10,6 +10,7 @@ HIP kernels choose their own launch shapes.
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -153,6 +154,13 @@ def fused_gemv_norm(raw, dtype, x: torch.Tensor, r: torch.Tensor | None, weight:
     return y
 
 
+@functools.lru_cache(maxsize=4096)
+def _scratch_bytes(dtype: int, n_rows: int, K: int, T: int) -> int:
+    """Bytes of scratch that the call uses, 0 where it runs on the VALU: a function of the sizes alone, asked once."""
+    lib = N.load()
+    return lib.nsx_gemv_workspace_bytes(dtype, n_rows, K, T) if lib.nsx_gemv_uses_workspace(dtype, n_rows, K, T) else 0
+
+
 def fused_gemv(raw, dtype, x: torch.Tensor, n_rows: int, K: int,
                out_dtype: torch.dtype = torch.float16, block_n: int = 16,
                num_warps: int = 2, bias: torch.Tensor | None = None,
@@ -203,9 +211,7 @@ def fused_gemv(raw, dtype, x: torch.Tensor, n_rows: int, K: int,
             args = (int(dtype), flat.data_ptr(), n_rows, K, xc.data_ptr(), N.act_dtype_code(xc.dtype), T, y.data_ptr(),
                     None if bias is None else bias.data_ptr(), None if resid is None else resid.data_ptr())
             # several tokens: scratch for the activation terms of the matrix-core path (stream-ordered, as y)
-            nws = 0
-            if T > 1 and lib.nsx_gemv_uses_workspace(int(dtype), n_rows, K, T):
-                nws = lib.nsx_gemv_workspace_bytes(int(dtype), n_rows, K, T)
+            nws = _scratch_bytes(int(dtype), n_rows, K, T) if T > 1 else 0
             if nws > 0:
                 ws = torch.empty(nws, dtype=torch.uint8, device=x2.device)
                 N.check(lib.nsx_fused_gemv_ws(*args, ws.data_ptr(), nws, s), "fused_gemv")

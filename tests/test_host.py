@@ -258,6 +258,26 @@ def test_parse_size_and_api_on_cpu(tmp_path):
         ns.model._ffn_block(torch.randn(1, 64), 0)
 
 
+def test_gemv_scratch_size_is_asked_once(monkeypatch):
+    """fused_gemv of several tokens asks the library for its scratch size once per (format, rows, K, tokens), also where
+    the answer is none."""
+    from nurostream_amd.compute import kernels
+    lib, asked = N.load(), []
+
+    class Counting:
+        def __getattr__(self, name):
+            asked.append(name)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(kernels.N, "load", Counting)
+    kernels._scratch_bytes.cache_clear()
+    for _ in range(3):
+        assert kernels._scratch_bytes(int(GGMLType.Q8_0), 4096, 4096, 8) == lib.nsx_gemv_workspace_bytes(8, 4096, 4096, 8) > 0
+        assert kernels._scratch_bytes(int(GGMLType.Q4_K), 512, 1024, 4) == 0
+    assert len(asked) == 3
+    kernels._scratch_bytes.cache_clear()
+
+
 def test_launch_caches(tmp_path):
     """csrc/launch_cache.h, compiled for the host: an answer is asked for once however many kernels and LDS sizes a
     process uses, from several threads; an LDS limit only grows, and an error is not remembered."""
