@@ -374,7 +374,7 @@ int nsx_dequantize_rows(int ggml_type, const void *raw, int64_t n_rows, int64_t 
 int nsx_rope_kv_append(float *qkv, const float *q_bias, const float *k_bias, const float *v_bias, int n_head,
                        int n_kv, int head_dim, const float *inv_freq, float amplitude, const int32_t *pos,
                        float *k_cache, float *v_cache, int64_t ctx_max, void *stream);
-/* Workspace bytes of nsx_attn_decode for this cache length. */
+/* Workspace bytes of nsx_attn_decode for this cache length (4-byte aligned). */
 int64_t nsx_attn_workspace_bytes(int n_head, int head_dim, int64_t ctx_max);
 /* model/gpt_oss.py:73-85 sink_attention for the query token at position
  * pos: keys 0..pos (the last `window` of them when window > 0), query head h

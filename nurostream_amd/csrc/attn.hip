@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
   __shared__ float ws[ATTN_MAX_SPLIT];
   __shared__ float red[4][ATTN_D];
   const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const float2* ml = (const float2*)(part + (int64_t)n_head * nsplit * ATTN_D) + (int64_t)h * nsplit;
+  const float* ml = part + ((int64_t)n_head * ATTN_D + 2 * h) * nsplit;  // (m, l) pairs; the workspace is 4-byte aligned
   const float sink = sinks ? sinks[h] : -INFINITY;
   const int p = *pos_ptr;
   if (p < 0 || p >= ctx_max) return;
@@ -387,7 +387,10 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(
   const int per = attn_per(total, nsplit, nw), nc = (total + per - 1) / per;  // 1 <= nc <= nsplit
   float2 v[LPS];
 #pragma unroll
-  for (int i = 0; i < LPS; ++i) v[i] = ml[min(lane + 64 * i, nc - 1)];
+  for (int i = 0; i < LPS; ++i) {
+    const float* p2 = ml + 2 * min(lane + 64 * i, nc - 1);
+    v[i] = float2{p2[0], p2[1]};
+  }
   float M = sink;
 #pragma unroll
   for (int i = 0; i < LPS; ++i) M = fmaxf(M, v[i].x);

@@ -152,6 +152,24 @@ def test_attention_split_edges(dev, heads, window):
         assert torch.equal(kv.v[0][:, p].cpu(), qkv.cpu().reshape(-1, 64)[H + G:])
 
 
+def test_attention_workspace_at_any_float(dev):
+    """The workspace needs no more than a float's alignment: the same bits with it 4, 8 and 12 bytes further on."""
+    from nurostream_amd.model.decode import DeviceKV, attn_decode
+    c = _cfg(n_head=8, n_kv=2, window=0)
+    kv = DeviceKV(1, c, 3000, dev)
+    g = torch.Generator().manual_seed(5)
+    kv.k[0].copy_(torch.randn(c.n_head_kv, 3000, 64, generator=g))
+    kv.v[0].copy_(torch.randn(c.n_head_kv, 3000, 64, generator=g))
+    kv.pos.fill_(2900)
+    q = torch.randn(c.n_head * 64, generator=g).to(dev)
+    out = attn_decode(q, kv, 0, None, 0, c)
+    n = kv.workspace.numel()
+    for off in (4, 8, 12):
+        kv.workspace = torch.empty(n + 16, dtype=torch.uint8, device=dev)[off:off + n]
+        assert kv.workspace.data_ptr() % 16 == off
+        assert torch.equal(attn_decode(q, kv, 0, None, 0, c), out), off
+
+
 @pytest.mark.parametrize("window", [0, 100, 1000])
 @pytest.mark.parametrize("sink", [True, False])
 def test_attention_keys_of_minus_infinity(dev, window, sink):
