@@ -197,8 +197,9 @@ typedef struct nsx_moe_layer {
 } nsx_moe_layer;
 
 /* Bytes of caller-provided workspace for T tokens. The caller zeroes the
- * workspace once before its first use (padding inside it must read as zero);
- * calls that share one workspace must not overlap. */
+ * workspace once before its first use (padding inside it must read as zero;
+ * calls of more tokens than one grouped pass takes need not: passes write all
+ * that they read of it); calls that share one workspace must not overlap. */
 int64_t nsx_moe_workspace_bytes(const nsx_moe_layer *L, int64_t T);
 /* The same for grouped passes of up to 8192 (token, expert) pairs, which
  * nsx_moe_forward and nsx_moe_forward_addnorm run where the workspace holds

@@ -118,15 +118,29 @@ class MoELayer:
         self._tiles = tabs  # keep the tables alive with the layer
 
     def workspace(self, T: int) -> torch.Tensor:
+        """The workspace of a call of T tokens: the layer's own, kept for calls of as many tokens, where one pass of the
+        kernels takes them all. Longer prompts run in passes, whose workspace is large (231 MB at 2880 x 2880, top-4) and
+        the same for every length: theirs is scratch of one call, stream-ordered from torch's allocator, so that it serves
+        every layer and length in turn; where the allocator has none for passes of 8192 (token, expert) pairs, passes of
+        4096."""
         ws = self._ws.get(T)
         if ws is None:
-            n = N.load().nsx_moe_workspace_bytes_wide(C.byref(self._c), T)
-            if n < 0:
-                raise ValueError(f"bad layer for T={T}")
+            narrow, wide = self._ws_bytes(T)
+            if wide > narrow:  # (grouped passes write all that they read of it: not zeroed)
+                try:
+                    return torch.empty(wide, dtype=torch.uint8, device=self.device)
+                except torch.cuda.OutOfMemoryError:
+                    return torch.empty(narrow, dtype=torch.uint8, device=self.device)
             # zeroed once: padding inside the workspace must read as zero
-            ws = torch.zeros(max(n, 256), dtype=torch.uint8, device=self.device)
-            self._ws[T] = ws
+            ws = self._ws[T] = torch.zeros(max(narrow, 256), dtype=torch.uint8, device=self.device)
         return ws
+
+    def _ws_bytes(self, T: int) -> tuple[int, int]:
+        lib, L = N.load(), C.byref(self._c)
+        narrow, wide = lib.nsx_moe_workspace_bytes(L, T), lib.nsx_moe_workspace_bytes_wide(L, T)
+        if narrow < 0 or wide < 0:
+            raise ValueError(f"bad layer for T={T}")
+        return narrow, wide
 
     def prompt_kernels(self, T: int) -> bool:
         """Whether T tokens run the kernels with work items of up to 64 tokens."""
@@ -342,10 +356,7 @@ class MoELayer:
 
     def new_workspace(self, T: int) -> torch.Tensor:
         """A separate zeroed workspace for T tokens (for phase runs that overlap)."""
-        n = N.load().nsx_moe_workspace_bytes(C.byref(self._c), T)
-        if n < 0:
-            raise ValueError(f"bad layer for T={T}")
-        return torch.zeros(max(n, 256), dtype=torch.uint8, device=self.device)
+        return torch.zeros(max(self._ws_bytes(T)[0], 256), dtype=torch.uint8, device=self.device)
 
 
 def router_topk(h: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, top_k: int,

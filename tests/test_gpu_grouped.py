@@ -360,6 +360,48 @@ def test_mx_prompt_kernel_bitwise(dev, n_embd, n_ff, T, bias, slabs):
     assert torch.equal(ip, ig) and torch.equal(op, og)
 
 
+@pytest.mark.parametrize("name,layout,dispatch", [("gptoss-small", "t64", "auto"), ("qwen3-small", "gguf", "auto"),
+                                                  ("qwen3-small", "gguf", "grouped")])
+def test_prompt_workspaces_are_scratch(dev, name, layout, dispatch, monkeypatch):
+    """Prompts of more than one pass of 4096 pairs: no layer keeps a workspace for them, at any length; what the memory
+    held before does not matter; and where the allocator has none for the wide passes, the narrow ones give the same
+    bits."""
+    from nurostream_amd import synth
+    cfg = _small(name)
+    layers = [_layer(cfg, synth.make_layer(cfg, seed=s, device=dev), layout, dispatch=dispatch) for s in (47, 48, 49)]
+    P = 4096 // cfg.top_k
+    # (last passes of P + 37, 2 and P + 37 tokens: "auto" runs 2 per pair; from 16 tokens on the router's sums are the same
+    # in passes of either size)
+    Ts = (P + 37, 2 * P + 2, 3 * P + 37)
+    h = synth.activations(Ts[-1], cfg.n_embd, seed=3, device=dev)
+    refs = [layer(h[:64])[0] for layer in layers]  # (everything else that a layer keeps)
+    del refs
+    torch.cuda.synchronize()
+    kept = torch.cuda.memory_allocated()
+    outs = [layer(h[:T])[0].clone() for layer in layers for T in Ts]
+    # (a block of the allocator's may be up to 1 MB larger than its tensor)
+    assert torch.cuda.memory_allocated() - kept <= sum(o.numel() * 4 + (1 << 20) for o in outs)
+    n = layers[0].workspace(Ts[-1]).numel()
+    junk = torch.full((2 * n + (64 << 20),), 255, dtype=torch.uint8, device=dev)  # every byte of the freed scratch
+    del junk
+    again = [layer(h[:T])[0].clone() for layer in layers for T in Ts]
+    assert all(torch.equal(a, b) for a, b in zip(outs, again))
+    narrow, wide = layers[0]._ws_bytes(Ts[-1])
+    assert wide > narrow
+    empty, sizes = torch.empty, []
+
+    def short(*a, **k):
+        if a and a[0] in (narrow, wide):
+            sizes.append(a[0])
+            if a[0] == wide:
+                raise torch.cuda.OutOfMemoryError("no memory for the wide passes")
+        return empty(*a, **k)
+
+    monkeypatch.setattr(torch, "empty", short)
+    out = layers[0](h)[0]
+    assert sizes == [wide, narrow] and torch.equal(out, outs[2])
+
+
 @pytest.mark.parametrize("name,layout,T", [("gptoss-small", "t64", 2100), ("qwen3-small", "gguf", 1030)])
 def test_wide_passes_equal_narrow_ones(dev, name, layout, T):
     """More than 8192 pairs in passes of 8192 (the workspace for it), of 4096 (the plain workspace), and the last pass."""
