@@ -612,15 +612,15 @@ int64_t nsx_gemv_mm_workspace(int t, int64_t n_rows, int64_t K, int64_t T) {
 // K x tokens where rows are few (a row's chain of units, once per 4 tokens) and in steps of its workgroups where K is
 // small; this one's starts at its two launches and a tile's way through LDS, longer for the K-quants' wide blocks and for
 // Q8_0 of 6 to 8 tokens (8 waves) outside K of 2048 .. 3072, where one pass of 12 units a wave holds all of it.
-//  2 tokens: rows x K. Q4_0 2880 x 2880 9.2 / 10.4, 5120 x 2880 13.4 / 12.1; Q4_K 5825 x 2816 14.3 / 16.3, 12288 x 4096
-//   31.8 / 20.9; Q6_K 8192 x 8192 38.7 / 35.1, 16384 x 4096 (two blocks a wave spill) 27.0 / 29.9, 32768 x 2048 29 / 23.
-//  3, 4: Q4_0, MXFP4 from 4 Mi weights on (2048 x 2048 11.3 / 9.6); Q8_0 1024 x 4096 10.0 / 12.1, 2048 x 2048 10.6 / 9.6;
-//   Q4_K 4096 x 1024 9.4 / 11.6, 2896 x 2048 13.4 / 13.1, 1448 x 4096 at 3 13.2 / 15.1, 512 x 8192 at 3 21 / 19.5.
+//  2 tokens: rows x K. Q4_0 2912 x 2880 9.4 / 10.1, 4119 x 2880 12.5 / 11.8; Q4_K 5825 x 2816 14.3 / 16.3, 8192 x 4096
+//   22.1 / 18.2; Q6_K 8192 x 8192 38.7 / 35.1, 16384 x 4096 (two blocks a wave spill) 27.0 / 29.9, 32768 x 2048 29 / 23.
+//  3, 4: Q4_0, MXFP4 from 4 Mi weights on (2048 x 2048 11.2 / 9.6); Q8_0 1024 x 4096 10.0 / 12.1, 2048 x 2048 10.7 / 9.6;
+//   Q4_K 4096 x 1024 9.4 / 11.6, 2896 x 2048 13.2 / 13.1, 1448 x 4096 at 3 13.2 / 15.1, 512 x 8192 at 3 21 / 19.5.
 //  5: Q4_0 1024 x 1024 7.6 / 8.5, 2048 x 512 7.3 / 8.1, 512 x 2048 11.0 / 9.4, 4096 x 256 8.9 / 8.0, 1448 x 1024 10 / 8.4;
 //   Q4_K 1024 x 2048 10.0 / 12.6, 728 x 2816 12.0 / 13.5, 512 x 4096 16.1 / 14.7; Q6_K 728 x 2816 11.1 / 14.0.
-//  6 to 8: MXFP4 1024 x 2048 10.1 / 10.7, 4096 x 256 11.7 / 8.1; Q8_0 1024 x 4096 at 6 18.3 / 20.6, at 8 24 / 20.5, 1024 x
+//  6 to 8: MXFP4 1024 x 2048 10.1 / 10.7, 4096 x 256 11.7 / 8.1; Q8_0 1024 x 4096 at 6 18.3 / 20.6, at 8 24 / 20.9, 1024 x
 //   2048 at 8 12.7 / 14.4, 1029 x 2880 21.9 / 12.4; Q4_K 2048 x 1024 at 6 12.6 / 13.0, 4096 x 512 10.9 / 11.7, 8192 x 256
-//   15.8 / 12.3; Q6_K 1448 x 1024 7.9 / 9.9, 4096 x 256 11.6 / 8.9.
+//   15.8 / 12.3; Q6_K 1448 x 1024 7.7 / 9.9, 4096 x 256 11.6 / 8.9.
 //  9 to 16: Q4_K 1024 x 1024 at 9 10.6 / 13.3, at 16 15 / 12; Q6_K the same, 9.7 / 10.9; the others gain from 1 Mi on.
 static bool gm_pays(int t, int64_t n_rows, int64_t K, int64_t T) {
   const double n = (double)n_rows * K / (1 << 20);
