@@ -305,7 +305,8 @@ def test_q4k_prompt_kernel_bitwise(dev, n_embd, n_ff):
 
 def test_q4k_gemm_kernel_bitwise(dev):
     """The same with a router that gives every token the same experts and weights in any batch: the outputs of
-    each token compared bit for bit between one call of 63 tokens and nine of 7."""
+    each token compared bit for bit between one call of 63 tokens and nine of 7 (16-token items: the layer is too small
+    for those of 64, test_q4k_prompt_kernel_bitwise)."""
     from nurostream_amd import synth
     cfg = _small("qwen3-small")
     t = synth.make_layer(cfg, seed=31, device=dev)
@@ -325,7 +326,8 @@ def test_q4k_gemm_kernel_bitwise(dev):
 def test_mx_gemm_kernel_bitwise(dev, n_embd, n_ff, T, bias, slabs):
     """Many tokens per expert (one expert with more than a work item, one with few): the same bits as the per-pair
     kernels, whose sums over K it repeats (top-4: those split the down product in 16 / top_k chunks, the grouped ones
-    in 4); experts in one tensor and at addresses of their own."""
+    in 4); experts in one tensor and at addresses of their own. (Layers too small for the prompt kernels:
+    test_mx_prompt_kernel_bitwise has those.)"""
     from nurostream_amd import synth
     cfg = synth.MoEConfig("mx", synth.GGMLType.MXFP4, 8, 4, n_embd, n_ff, "gptoss",
                           "clamped_swiglu" if bias else "silu_mul", bias, torch.bfloat16)
